@@ -84,6 +84,64 @@ FX_HD void st_hint(cx<T>* p, cx<T> w)
     }
 }
 
+// Read-only window onto a workgroup's part of a buffer.  On the device it is a buffer resource
+// in SGPRs: a load takes a 32-bit per-lane byte offset and a scalar one, so a thread keeps one
+// offset register for all the planes it walks, and a lane whose offset is kNone (past every
+// window) reads zero without touching memory, where a clamped global load would fetch again.
+template <typename T>
+struct Window {
+    static constexpr unsigned kNone = 0x80000000u;
+#if defined(__HIP_DEVICE_COMPILE__)
+    __amdgpu_buffer_rsrc_t r;
+    __device__ __forceinline__ Window(const cx<T>* p, int elems)
+        : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<cx<T>*>(p), (short)0,
+                                              elems * (int)sizeof(cx<T>), 0x00027000))
+    {
+    }
+    // `lane` per lane, `uni` the same for the wave, both in bytes.
+    __device__ __forceinline__ cx<T> ld(unsigned lane, unsigned uni) const
+    {
+        if constexpr (sizeof(T) == 8) {
+            using V4 = unsigned __attribute__((ext_vector_type(4)));
+            return __builtin_bit_cast(
+                cx<T>, (V4)__builtin_amdgcn_raw_buffer_load_b128(r, (int)lane, (int)uni, 0));
+        } else {
+            using V2 = unsigned __attribute__((ext_vector_type(2)));
+            return __builtin_bit_cast(
+                cx<T>, (V2)__builtin_amdgcn_raw_buffer_load_b64(r, (int)lane, (int)uni, 0));
+        }
+    }
+#else
+    const cx<T>* p;
+    unsigned bytes;
+    FX_HD Window(const cx<T>* q, int elems) : p(q), bytes((unsigned)elems * sizeof(cx<T>)) {}
+    FX_HD cx<T> ld(unsigned lane, unsigned uni) const
+    {
+        if (lane >= bytes || lane + uni >= bytes) return cx<T>{T(0), T(0)};
+        return p[(lane + uni) / sizeof(cx<T>)];
+    }
+#endif
+};
+
+// No instruction is scheduled across this point (the compiler otherwise gathers the loads or
+// LDS reads of later groups in front of this one's arithmetic, or puts them off behind it).
+FX_HD void sched_fence()
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_sched_barrier(0);
+#endif
+}
+
+// The value is computed here: neither sunk to its use in a later block nor put off behind the
+// loads that follow.
+template <typename T>
+FX_HD void settle(cx<T>& a)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(a.r), "+v"(a.i));
+#endif
+}
+
 // Line lengths that have a W table in the bank, in bank order.
 constexpr int kLens[] = {2, 3, 4, 6, 8, 9, 12, 16, 17, 24, 36, 48};
 constexpr int kNumLens = sizeof(kLens) / sizeof(kLens[0]);

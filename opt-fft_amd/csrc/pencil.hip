@@ -35,19 +35,18 @@ namespace fx {
           "pencil_" #N0 "x" #N1 "x" #N2 "_" TAG "_bwd_s" #SPW "t" #NT "b" #NTB "c" #CH "p" #PIPE SUF "_r1")
 
 // Residue-split single pass (xres.hpp): "xres_<shape>_<prec>_<dir>_v1r<R>t<NT>", R workgroups
-// per volume, each holding N0 / R x-planes in LDS.
-#define FX_X(N0, N1, N2, T, S, R, NT, OR, NAME) \
-    r.push_back(xres_desc<XResCfg<N0, N1, N2, T, S, R, NT, OR>>(NAME))
-#define FX_X_BOTH(N0, N1, N2, T, TAG, R, NT)                                                       \
-    FX_X(N0, N1, N2, T, -1, R, NT, 0, "xres_" #N0 "x" #N1 "x" #N2 "_" TAG "_fwd_v1r" #R "t" #NT); \
-    FX_X(N0, N1, N2, T, +1, R, NT, 0, "xres_" #N0 "x" #N1 "x" #N2 "_" TAG "_bwd_v1r" #R "t" #NT)
+// per volume, each holding N0 / R x-planes in LDS; PF groups of loads in flight.
+#define FX_X(N0, N1, N2, T, S, R, NT, OR, PF, NAME) \
+    r.push_back(xres_desc<XResCfg<N0, N1, N2, T, S, R, NT, OR, PF>>(NAME))
+#define FX_X_BOTH(N0, N1, N2, T, TAG, R, NT, PF)                                                  \
+    FX_X(N0, N1, N2, T, -1, R, NT, 0, PF, "xres_" #N0 "x" #N1 "x" #N2 "_" TAG "_fwd_v1r" #R "t" #NT); \
+    FX_X(N0, N1, N2, T, +1, R, NT, 0, PF, "xres_" #N0 "x" #N1 "x" #N2 "_" TAG "_bwd_v1r" #R "t" #NT)
 // "o<OR>": the x pass's point order (XResCfg OR: 1 rotated thread blocks, 2 offset starts).
-#define FX_XO_BOTH(N0, N1, N2, T, TAG, R, NT, OR)                                                \
-    FX_X(N0, N1, N2, T, -1, R, NT, OR,                                                          \
+#define FX_XO_BOTH(N0, N1, N2, T, TAG, R, NT, OR, PF)                                           \
+    FX_X(N0, N1, N2, T, -1, R, NT, OR, PF,                                                      \
          "xres_" #N0 "x" #N1 "x" #N2 "_" TAG "_fwd_v1r" #R "t" #NT "o" #OR);                   \
-    FX_X(N0, N1, N2, T, +1, R, NT, OR,                                                          \
+    FX_X(N0, N1, N2, T, +1, R, NT, OR, PF,                                                      \
          "xres_" #N0 "x" #N1 "x" #N2 "_" TAG "_bwd_v1r" #R "t" #NT "o" #OR)
-
 // (Pass B with plain stores, PencilCfg XH = 1, measured 8% slower at 36^3 x 128 and 1% at
 // 24x24x48 x 64 than with nontemporal ones: not registered.)
 
@@ -99,26 +98,31 @@ void register_pencil(std::vector<KernelDesc>& r)
     // were issued one or two at a time, and issuing them together spilled.  A second form
     // (512 threads, 169 VGPRs: two-stage 4 x 9 line passes, loads six at a time, offset
     // starts) ran without scratch but took 69.8 us at x 128 and 251.4 at x 512 against 57.0 /
-    // 225.3 us for the one-task form.  Not kept.
-    FX_XO_BOTH(36, 36, 36, double, "c128", 6, 512, 2);
-    FX_XO_BOTH(36, 36, 36, double, "c128", 6, 512, 1);
-    FX_X_BOTH(36, 36, 36, double, "c128", 6, 512);
-    FX_X_BOTH(36, 36, 36, double, "c128", 6, 256);
-    FX_XO_BOTH(24, 24, 48, double, "c128", 4, 384, 2);
-    FX_X_BOTH(24, 24, 48, double, "c128", 4, 384);
-    FX_X_BOTH(24, 24, 48, double, "c128", 4, 256);
-    FX_XO_BOTH(24, 24, 24, double, "c128", 3, 256, 1);
-    FX_X_BOTH(24, 24, 24, double, "c128", 3, 256);
-    FX_X_BOTH(24, 24, 24, double, "c128", 3, 192);
-    FX_X_BOTH(24, 24, 24, double, "c128", 4, 192);
+    // 225.3 us for the one-task form.  Not kept.  (The figures above are from before the x
+    // pass was pipelined, xres.hpp; since then 24x24x48 x 64 takes 16.4 us with rotated blocks
+    // (o1) and 16.7 with offset starts, and 24^3 x 8 6.0 us in six workgroups (r6) against 6.6
+    // in four, which is the better one from x 64 on.)
+    FX_XO_BOTH(36, 36, 36, double, "c128", 6, 512, 2, 4);
+    FX_XO_BOTH(36, 36, 36, double, "c128", 6, 512, 1, 4);
+    FX_X_BOTH(36, 36, 36, double, "c128", 6, 512, 4);
+    FX_X_BOTH(36, 36, 36, double, "c128", 6, 256, 4);
+    FX_XO_BOTH(24, 24, 48, double, "c128", 4, 384, 1, 2);
+    FX_XO_BOTH(24, 24, 48, double, "c128", 4, 384, 2, 2);
+    FX_X_BOTH(24, 24, 48, double, "c128", 4, 384, 2);
+    FX_X_BOTH(24, 24, 48, double, "c128", 4, 256, 2);
+    FX_XO_BOTH(24, 24, 24, double, "c128", 3, 256, 1, 3);
+    FX_X_BOTH(24, 24, 24, double, "c128", 3, 256, 3);
+    FX_X_BOTH(24, 24, 24, double, "c128", 3, 192, 4);
+    FX_X_BOTH(24, 24, 24, double, "c128", 4, 192, 4);
+    FX_X_BOTH(24, 24, 24, double, "c128", 6, 192, 4);
     // complex64: 24x24x48 x 256 r2 (12 planes, 112.9 KB) 28.8 us and r3 31.6 us against 42.0 us
     // for the best pencil (x 64: 12.6 / 14.0 against 17.1 us); 36^3 x 512 r3 125.7 us against
     // 94.0 us for the split-resident kernel (r4 161.3, r6 134.6), but at x 64 r3 20.5 against
     // 21.6 us for the pencil.
-    FX_X_BOTH(24, 24, 48, float, "c64", 2, 384);
-    FX_X_BOTH(24, 24, 48, float, "c64", 3, 256);
-    FX_XO_BOTH(36, 36, 36, float, "c64", 3, 512, 2);
-    FX_X_BOTH(36, 36, 36, float, "c64", 3, 512);
+    FX_X_BOTH(24, 24, 48, float, "c64", 2, 384, 3);
+    FX_X_BOTH(24, 24, 48, float, "c64", 3, 256, 3);
+    FX_XO_BOTH(36, 36, 36, float, "c64", 3, 512, 2, 2);
+    FX_X_BOTH(36, 36, 36, float, "c64", 3, 512, 2);
 }
 
 }  // namespace fx

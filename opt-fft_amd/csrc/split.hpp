@@ -46,15 +46,6 @@ struct SplitCfg {
     static_assert(N0 % R == 0, "the rounds split the x-planes evenly");
 };
 
-// No instruction is scheduled across this point (the groups of a two-stage line would
-// otherwise have their LDS reads hoisted together, holding all N points in registers).
-FX_HD void sched_fence()
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-    __builtin_amdgcn_sched_barrier(0);
-#endif
-}
-
 // Line DFT of N = A * B points in LDS (point n at b0 + n * st), in two stages that hold A,
 // then B, points in registers instead of N (Cooley-Tukey over n = a * B + b):
 //   stage 1, for each b: DFT_A over a of x[a * B + b], times W_N^(b * k1), written back to

@@ -13,8 +13,17 @@
 // once; it is read R times, by the R workgroups of its volume, which are consecutive
 // workgroups of one XCD (an 8-XCD part dispatches workgroup g to XCD g mod 8), so they run
 // together and most reads of a line after the first are served by that XCD's L2.  The
-// inputs are therefore read with plain loads (HL = 0), the outputs stored nontemporal
-// (HS = 1).  What bounds the kernel is the rate at which one CU reads from L2.
+// inputs are therefore read with plain loads, the outputs stored nontemporal (HS = 1).
+//
+// The x pass is one stream of groups of M loads (M planes at one point) with PF groups in
+// flight across the points of a thread, its order pinned by sched_fence: left to itself the
+// compiler waits for all loads of a point before it issues the next ones (14, 13 and 9 at a
+// time at 36^3), and recomputes 64-bit addresses for each.  Against that form 24^3 x 365
+// takes 36.7 us instead of 39.9 (r3), 24x24x48 complex64 x 300 36.7 instead of 40.6 (r3),
+// 36^3 x 64 33.4 instead of 35.0 (r6).  At 36^3 x 128 it gains nothing (56.3 against 56.9):
+// the rate at which a CU reads from L2 bounds that x pass, whatever is in flight (PF = 2 .. 6
+// 56.3-57.3 us).  A probe that only reads (R = 6, every workgroup all of its volume) gets
+// 62-75 GB/s a CU there, 108 from an L2 that already holds the volumes.
 #pragma once
 
 #include "kernels.hpp"
@@ -26,15 +35,16 @@ namespace fx {
 // thread block h mod PPT (the blocks of NT points taken in rotated order); 2: residue h
 // starts at point h * PLANE / R (the plane walked with a wrap).  1 and 2 spread the R
 // workgroups' requests over different lines (and L2 channels) at the price of keeping each
-// line in L2 longer.
+// line in L2 longer.  PF: groups of M loads in flight (24-32 loads; 12 where a 48-point line
+// sets the VGPRs: PF = 4 took 17.1 us at 24x24x48 x 64, PF = 2 16.7).
 template <int N0_, int N1_, int N2_, typename T_, int S_, int R_, int NT_, int OR_ = 0,
-          int PZ_ = 1, int HL_ = 0, int HS_ = 1, int ALG_ = 0>
+          int PF_ = 4, int PZ_ = 1, int HS_ = 1, int ALG_ = 0>
 struct XResCfg {
     using T = T_;
     static constexpr int N0 = N0_, N1 = N1_, N2 = N2_, S = S_, R = R_, NT = NT_, PZ = PZ_;
-    static constexpr int OR = OR_;
+    static constexpr int OR = OR_, PF = PF_;
     static constexpr int PPT = (N1 * N2 + NT - 1) / NT;   // (y, z) points per thread
-    static constexpr int HL = HL_, HS = HS_, ALG = ALG_, V17 = ALG_, VPW = 1, P = 0;
+    static constexpr int HS = HS_, ALG = ALG_, V17 = ALG_, VPW = 1, P = 0;
     static_assert(N0 % R == 0, "the residues split the x-planes evenly");
     static constexpr int M = N0 / R;       // x-planes per workgroup
     static constexpr int V = N0 * N1 * N2;
@@ -73,43 +83,89 @@ struct XRes {
     static FX_HD void xpass(int tid, long v, int h, const cx<T>* __restrict__ in, cx<T>* sm,
                             const Bank<T>* __restrict__ bk)
     {
-        const cx<T>* __restrict__ src = in + v * (long)C::V;
+        // Waves whose points of the last block all lie past the plane leave it out.
+        const bool last = wave_first(tid) + (C::PPT - 1) * C::NT < C::PLANE;
+        if (C::PPT == 1 || last) xrun<C::PPT>(tid, v, h, in, sm, bk);
+        else xrun<C::PPT == 1 ? 1 : C::PPT - 1>(tid, v, h, in, sm, bk);
+    }
+    // Point of the kk-th of NK thread blocks, or PLANE and above past the end.
+    template <int NK>
+    static FX_HD int point(int tid, int h, int kk)
+    {
+        if constexpr (C::OR == 1) return tid + ((kk + h) % NK) * C::NT;
+        const int p = tid + kk * C::NT;
+        if constexpr (C::OR == 2) {
+            if (p >= C::PLANE) return p;
+            const int w = p + h * (C::PLANE / C::R);
+            return w < C::PLANE ? w : w - C::PLANE;
+        }
+        return p;
+    }
+    // First thread of tid's wave.
+    static FX_HD int wave_first(int tid)
+    {
+#if defined(__HIP_DEVICE_COMPILE__)
+        return __builtin_amdgcn_readfirstlane(tid & ~63);
+#else
+        return tid & ~63;
+#endif
+    }
+    // NK blocks of points as one stream of NK * R groups of M loads (group (kk, m): planes
+    // M m .. M m + M - 1 at point kk), PF groups in flight.
+    template <int NK>
+    static FX_HD void xrun(int tid, long v, int h, const cx<T>* __restrict__ in, cx<T>* sm,
+                           const Bank<T>* __restrict__ bk)
+    {
+        constexpr int E = (int)sizeof(cx<T>), NG = NK * C::R;
+        constexpr int PF = C::PF < NG ? C::PF : NG;
+        const Window<T> win(in + v * (long)C::V, C::V);
         cx<T> wr[C::R], tw[C::M];
 #pragma unroll
         for (int m = 1; m < C::R; ++m) wr[m] = w0(C::M * ((m * h) % C::R), bk);
 #pragma unroll
         for (int n = 1; n < C::M; ++n) tw[n] = w0(n * h, bk);
-        for (int kk = 0; kk < C::PPT; ++kk) {
-            int p;
-            if constexpr (C::OR == 1) {
-                p = tid + ((kk + h) % C::PPT) * C::NT;
-                if (p >= C::PLANE) continue;
-            } else {
-                p = tid + kk * C::NT;
-                if (p >= C::PLANE) continue;
-                if constexpr (C::OR == 2) {
-                    p += h * (C::PLANE / C::R);
-                    p = p < C::PLANE ? p : p - C::PLANE;
+        unsigned off[NK];
+#pragma unroll
+        for (int kk = 0; kk < NK; ++kk) {
+            const int p = point<NK>(tid, h, kk);
+            off[kk] = p < C::PLANE ? (unsigned)(p * E) : Window<T>::kNone;
+        }
+        cx<T> buf[PF][C::M], a[C::M];
+#pragma unroll
+        for (int g = 0; g < PF; ++g)
+#pragma unroll
+            for (int n = 0; n < C::M; ++n)
+                buf[g][n] = win.ld(off[g / C::R], (unsigned)((n + C::M * (g % C::R)) * C::PLANE * E));
+        sched_fence();
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const int m = g % C::R, f = g + PF;
+#pragma unroll
+            for (int n = 0; n < C::M; ++n)
+                a[n] = m == 0 ? buf[g % PF][n] : a[n] + cmul(buf[g % PF][n], wr[m]);
+            if (m > 0) {
+#pragma unroll
+                for (int n = 0; n < C::M; ++n) settle(a[n]);
+            }
+            if (f < NG) {
+#pragma unroll
+                for (int n = 0; n < C::M; ++n)
+                    buf[f % PF][n] =
+                        win.ld(off[f / C::R], (unsigned)((n + C::M * (f % C::R)) * C::PLANE * E));
+            }
+            if (m == C::R - 1) {
+#pragma unroll
+                for (int n = 1; n < C::M; ++n) a[n] = cmul(a[n], tw[n]);
+                dft<C::M, C::S, T, C::ALG>(a, bk);
+                const int p = (int)(off[g / C::R] / E);
+                if (p < C::PLANE) {
+                    const int y = p / C::N2;
+                    const int z = p - y * C::N2;
+#pragma unroll
+                    for (int q = 0; q < C::M; ++q) sm[q * C::SS + y * C::YS + z] = a[q];
                 }
             }
-            cx<T> a[C::M];
-#pragma unroll
-            for (int n = 0; n < C::M; ++n) a[n] = ld_hint<C::HL>(src + n * C::PLANE + p);
-#pragma unroll
-            for (int m = 1; m < C::R; ++m) {
-#pragma unroll
-                for (int n = 0; n < C::M; ++n) {
-                    const cx<T> x = ld_hint<C::HL>(src + (n + C::M * m) * C::PLANE + p);
-                    a[n] = a[n] + cmul(x, wr[m]);
-                }
-            }
-#pragma unroll
-            for (int n = 1; n < C::M; ++n) a[n] = cmul(a[n], tw[n]);
-            dft<C::M, C::S, T, C::ALG>(a, bk);
-            const int y = p / C::N2;
-            const int z = p - y * C::N2;
-#pragma unroll
-            for (int q = 0; q < C::M; ++q) sm[q * C::SS + y * C::YS + z] = a[q];
+            sched_fence();
         }
     }
     // Phase 2: z lines (plane s, y).
