@@ -7,13 +7,13 @@
 // so the arrays stay in VGPRs and the twiddle reads are scalar loads from the bank.
 //   2, 3, 4    butterflies (3 is the Winograd form: one real scale by -1/2, one by sqrt(3)/2)
 //   8, 9, 16   Cooley-Tukey N1 x N2 with bank twiddles W_N^(n2 k1)
-//   6, 12, 24, 36, 48   Good-Thomas prime-factor (2x3, 4x3, 8x3, 4x9, 16x3): no twiddles,
+//   6, 12, 18, 24, 36, 48   Good-Thomas prime-factor (2x3, 4x3, 2x9, 8x3, 4x9, 16x3): no twiddles,
 //              the Ruritanian input map n = (N2 n1 + N1 n2) mod N and CRT output map
 //              k = (E1 k1 + E2 k2) mod N are pure register renaming
 //              (index maps as in bench/geom/strategies/L36_pfa.md:10-24)
 // The fourth parameter (V17) selects the line algorithm: for 17 as below; for the composite
 // lengths 1 takes the factors in the other order (8 = 4x2, 16 = 2x8, 6 = 3x2, 12 = 3x4,
-// 24 = 3x8, 36 = 9x4, 48 = 3x16), a radix order the create-time race can choose.
+// 18 = 9x2, 24 = 3x8, 36 = 9x4, 48 = 3x16), a radix order the create-time race can choose.
 //   17         V17 = 0: Rader with generator 3 -- a 16-point cyclic convolution done as two
 //              forward DFT16s and a pointwise product with the plan-time spectrum
 //              (construction of bench/geom/strategies/L17_rader.md:21-55);
@@ -292,6 +292,9 @@ FX_HD void dft(cx<T>* x, const Bank<T>* __restrict__ bk)
     } else if constexpr (N == 17) {
         if constexpr (V17 == 0) rader17<S>(x, bk);
         else fold17<S>(x, bk);
+    } else if constexpr (N == 18) {
+        if constexpr (V17 == 0) pfa<2, 9, S>(x, bk);
+        else pfa<9, 2, S>(x, bk);
     } else if constexpr (N == 24) {
         if constexpr (V17 == 0) pfa<8, 3, S>(x, bk);
         else pfa<3, 8, S>(x, bk);

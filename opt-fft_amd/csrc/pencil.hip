@@ -5,6 +5,7 @@
 // "_st" pass A with staggered HBM traffic (PencilCfg ST = 1).  Also the residue-split
 // single-pass kernels of the same geometries (xres.hpp): "xres_..._v1r<R>t<NT>".
 #include "kernels.hpp"
+#include "xhold.hpp"
 #include "xres.hpp"
 
 namespace fx {
@@ -47,6 +48,16 @@ namespace fx {
          "xres_" #N0 "x" #N1 "x" #N2 "_" TAG "_fwd_v1r" #R "t" #NT "o" #OR);                   \
     FX_X(N0, N1, N2, T, +1, R, NT, OR, PF,                                                      \
          "xres_" #N0 "x" #N1 "x" #N2 "_" TAG "_bwd_v1r" #R "t" #NT "o" #OR)
+// The same with most of the planes in registers (xhold.hpp): "...h<PR>", PR planes in LDS at a
+// time, PF groups of GS loads in flight.
+#define FX_XH(N0, N1, N2, T, S, R, NT, PR, GS, PF, NAME) \
+    r.push_back(xhold_desc<XHoldCfg<N0, N1, N2, T, S, R, NT, PR, GS, PF>>(NAME))
+#define FX_XH_BOTH(N0, N1, N2, T, TAG, R, NT, PR, GS, PF)                                        \
+    FX_XH(N0, N1, N2, T, -1, R, NT, PR, GS, PF,                                                  \
+          "xres_" #N0 "x" #N1 "x" #N2 "_" TAG "_fwd_v1r" #R "t" #NT "h" #PR);                    \
+    FX_XH(N0, N1, N2, T, +1, R, NT, PR, GS, PF,                                                  \
+          "xres_" #N0 "x" #N1 "x" #N2 "_" TAG "_bwd_v1r" #R "t" #NT "h" #PR)
+
 // (Pass B with plain stores, PencilCfg XH = 1, measured 8% slower at 36^3 x 128 and 1% at
 // 24x24x48 x 64 than with nontemporal ones: not registered.)
 
@@ -123,6 +134,11 @@ void register_pencil(std::vector<KernelDesc>& r)
     FX_X_BOTH(24, 24, 48, float, "c64", 3, 256, 3);
     FX_XO_BOTH(36, 36, 36, float, "c64", 3, 512, 2, 2);
     FX_X_BOTH(36, 36, 36, float, "c64", 3, 512, 2);
+    FX_XH_BOTH(36, 36, 36, double, "c128", 2, 256, 6, 9, 3);
+    FX_XH_BOTH(36, 36, 36, double, "c128", 4, 448, 6, 9, 2);
+    FX_XH_BOTH(24, 24, 48, double, "c128", 2, 256, 8, 6, 4);
+    FX_XH_BOTH(24, 24, 24, double, "c128", 2, 256, 8, 6, 4);
+    FX_XH_BOTH(24, 24, 48, float, "c64", 1, 384, 12, 6, 4);
 }
 
 }  // namespace fx
