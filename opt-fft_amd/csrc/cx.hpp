@@ -84,6 +84,20 @@ FX_HD void st_hint(cx<T>* p, cx<T> w)
     }
 }
 
+// 16 bytes of consecutive elements at t to p, which is aligned to one element.
+template <int H, typename T>
+FX_HD void st_wide(cx<T>* p, const cx<T>* t)
+{
+    if constexpr (sizeof(cx<T>) == 16) {
+        st_hint<H>(p, *t);
+    } else {
+        using V4 = T __attribute__((ext_vector_type(4), aligned(sizeof(cx<T>))));
+        const V4 w = {t[0].r, t[0].i, t[1].r, t[1].i};
+        if constexpr (H != 0) __builtin_nontemporal_store(w, reinterpret_cast<V4*>(p));
+        else *reinterpret_cast<V4*>(p) = w;
+    }
+}
+
 // Read-only window onto a workgroup's part of a buffer.  On the device it is a buffer resource
 // in SGPRs: a load takes a 32-bit per-lane byte offset and a scalar one, so a thread keeps one
 // offset register for all the planes it walks, and a lane whose offset is kNone (past every

@@ -58,6 +58,15 @@ namespace fx {
     FX_XH(N0, N1, N2, T, +1, R, NT, PR, GS, PF,                                                  \
           "xres_" #N0 "x" #N1 "x" #N2 "_" TAG "_bwd_v1r" #R "t" #NT "h" #PR)
 
+// "...h<PR>l": stored by a copy of 16 bytes a lane out of LDS (XHoldCfg LIN).
+#define FX_XHL(N0, N1, N2, T, S, R, NT, PR, GS, PF, NAME) \
+    r.push_back(xhold_desc<XHoldCfg<N0, N1, N2, T, S, R, NT, PR, GS, PF, 1>>(NAME))
+#define FX_XHL_BOTH(N0, N1, N2, T, TAG, R, NT, PR, GS, PF)                                       \
+    FX_XHL(N0, N1, N2, T, -1, R, NT, PR, GS, PF,                                                 \
+           "xres_" #N0 "x" #N1 "x" #N2 "_" TAG "_fwd_v1r" #R "t" #NT "h" #PR "l");               \
+    FX_XHL(N0, N1, N2, T, +1, R, NT, PR, GS, PF,                                                 \
+           "xres_" #N0 "x" #N1 "x" #N2 "_" TAG "_bwd_v1r" #R "t" #NT "h" #PR "l")
+
 // (Pass B with plain stores, PencilCfg XH = 1, measured 8% slower at 36^3 x 128 and 1% at
 // 24x24x48 x 64 than with nontemporal ones: not registered.)
 
@@ -130,15 +139,39 @@ void register_pencil(std::vector<KernelDesc>& r)
     // for the best pencil (x 64: 12.6 / 14.0 against 17.1 us); 36^3 x 512 r3 125.7 us against
     // 94.0 us for the split-resident kernel (r4 161.3, r6 134.6), but at x 64 r3 20.5 against
     // 21.6 us for the pencil.
+    // Small batches, where a workgroup's x pass (all of its volume from L2, at up to 108 GB/s a
+    // CU) and its line passes are latencies in a row: more residues shorten the line passes.
+    // 36^3 x 5 r12 11.4 us (r9 12.1, r6 12.8, pencil 11.9), x 16 13.4 against 15.6 (pencil);
+    // 24x24x48 x 8 r8 8.8 us (r4 10.5, pencil 10.0), x 32 11.2 against 13.0 (r4).
+    FX_XO_BOTH(36, 36, 36, double, "c128", 12, 256, 1, 4);
+    FX_XO_BOTH(24, 24, 48, double, "c128", 8, 256, 1, 4);
     FX_X_BOTH(24, 24, 48, float, "c64", 2, 384, 3);
     FX_X_BOTH(24, 24, 48, float, "c64", 3, 256, 3);
     FX_XO_BOTH(36, 36, 36, float, "c64", 3, 512, 2, 2);
     FX_X_BOTH(36, 36, 36, float, "c64", 3, 512, 2);
+    // Small batches again: 36^3 complex64 x 8 r12 10.7 us (r6 11.2, pencil 11.5), x 32 r6 13.7
+    // (r3 15.9); 24x24x48 complex64 x 9 r6 8.2 (r3 9.6), x 32 10.3 (11.2).  24^3 complex64
+    // against the LDS-resident kernel (one 576-thread workgroup a volume, one per CU): x 18
+    // r6 5.4 against 9.8 us, x 90 r2 8.1 against 10.3, x 300 r3 18.9 against 22.5; x 180, one
+    // volume for most CUs, 12.9 against 11.4.
+    FX_XO_BOTH(36, 36, 36, float, "c64", 6, 448, 2, 4);
+    FX_XO_BOTH(36, 36, 36, float, "c64", 12, 256, 1, 4);
+    FX_X_BOTH(24, 24, 48, float, "c64", 6, 192, 4);
+    FX_X_BOTH(24, 24, 24, float, "c64", 2, 320, 2);
+    FX_X_BOTH(24, 24, 24, float, "c64", 3, 192, 4);
+    FX_X_BOTH(24, 24, 24, float, "c64", 6, 192, 6);
+#define TT(N0,N1,N2,T,TAG,R,NT,PR,GS,PF,LIN) \
+    r.push_back(xhold_desc<XHoldCfg<N0,N1,N2,T,-1,R,NT,PR,GS,PF,LIN>>("T" #N0 "x" #N1 "x" #N2 TAG "r" #R "t" #NT "h" #PR "g" #GS "f" #PF "l" #LIN));
     FX_XH_BOTH(36, 36, 36, double, "c128", 2, 256, 6, 9, 3);
     FX_XH_BOTH(36, 36, 36, double, "c128", 4, 448, 6, 9, 2);
     FX_XH_BOTH(24, 24, 48, double, "c128", 2, 256, 8, 6, 4);
     FX_XH_BOTH(24, 24, 24, double, "c128", 2, 256, 8, 6, 4);
     FX_XH_BOTH(24, 24, 48, float, "c64", 1, 384, 12, 6, 4);
+    FX_XH_BOTH(24, 24, 24, float, "c64", 1, 192, 8, 6, 4);
+    FX_XHL_BOTH(24, 24, 24, float, "c64", 1, 192, 8, 6, 4);
+    FX_XHL_BOTH(36, 36, 36, float, "c64", 1, 448, 12, 9, 4);
+    FX_XHL_BOTH(36, 36, 36, float, "c64", 2, 256, 6, 9, 4);
+    FX_XHL_BOTH(36, 36, 36, float, "c64", 2, 448, 9, 9, 3);
 }
 
 }  // namespace fx

@@ -17,12 +17,24 @@
 //                      workgroups a volume fill the device there
 //   24^3 x 365, r2h8   36.7 -> 32.4 us (two workgroups per CU, 4 of 12 planes held)
 //   24x24x48 complex64 x 256, r1h12  28.9 -> 24.6 us (a volume per workgroup)
+//   24^3 complex64 x 678, r1h8l  37.4 (LDS-resident, one volume a CU) -> 30.9 us with four
+//                      workgroups per CU; x 1989 102.7 -> 88.0
+//   36^3 complex64 x 255, r1h12l  45.8 (split-resident) -> 40.8 us, x 589 123.3 -> 108.6;
+//                      r2h9l x 128 37.3 -> 25.5 us
 // At R = 2 a copy with the same reads, the same stores and no arithmetic takes 37.5 us at
 // 36^3 x 128: reads and stores come in turns, since the one round of workgroups walks in step.
 // The two workgroups of a volume walk it in the same order (19.6 us for the reads alone);
 // starts a plane part apart, which XRes needs at R = 6, read it at 29.4.
 // Stores are nontemporal: with plain ones 36^3 x 128 takes 50.8 us.  PR = 7 (42.5-43.0 us) and
 // 5 (41.2) against 6; 27 loads in flight, 18-36 being within 1%.
+//
+// LIN = 1: the y pass writes its lines back to LDS and a copy stores the planes, 16 bytes a
+// lane, where rows are not whole 128-byte lines and an element is 8 bytes: stores of 288-byte
+// rows at 36^3 complex64 took 27 us for 95 MB (49.0 us in all), the copy's 40.8.  With rows of
+// 576 (36^3 complex128: 44.7 against 40.5 us) or 384 bytes (24x24x48 complex64: 27.2 against
+// 24.6) the extra LDS round trip costs more than it gains; at 24^3 complex64 (192) it gains
+// from about 500 volumes on, 30.9 against 33.1 us at x 678, and loses at x 300, 22.1 against
+// 20.1, so both are raced.
 #pragma once
 
 #include <type_traits>
@@ -32,13 +44,13 @@
 
 namespace fx {
 
-// GS: planes per group of loads; PF: groups in flight during the x pass.
+// GS: planes per group of loads; PF: groups in flight during the x pass; LIN: see above.
 template <int N0_, int N1_, int N2_, typename T_, int S_, int R_, int NT_, int PR_, int GS_, int PF_,
-          int HS_ = 1, int PZ_ = 1, int ALG_ = 0>
+          int LIN_ = 0, int HS_ = 1, int PZ_ = 1, int ALG_ = 0>
 struct XHoldCfg {
     using T = T_;
     static constexpr int N0 = N0_, N1 = N1_, N2 = N2_, S = S_, R = R_, NT = NT_, PR = PR_;
-    static constexpr int GS = GS_, PF = PF_, HS = HS_, PZ = PZ_, ALG = ALG_, V17 = ALG_;
+    static constexpr int GS = GS_, PF = PF_, LIN = LIN_, HS = HS_, PZ = PZ_, ALG = ALG_, V17 = ALG_;
     static constexpr int M = N0 / R;                    // output x-planes per workgroup
     static constexpr int V = N0 * N1 * N2;
     static constexpr int PLANE = N1 * N2;
@@ -164,23 +176,44 @@ struct XHold {
             },
             bk);
     }
-    // y lines, LDS -> output x-planes R (rd PR + s) + h (rows of N2 elements, in order).
+    // y lines, LDS -> output x-planes R (rd PR + s) + h (rows of N2 elements, in order); LIN = 1:
+    // back to LDS, for copy.
     template <int rd>
-    static FX_HD void ypass(int tid, long v, int h, const cx<T>* sm, cx<T>* __restrict__ out,
+    static FX_HD void ypass(int tid, long v, int h, cx<T>* sm, cx<T>* __restrict__ out,
                             const Bank<T>* __restrict__ bk, T scl)
     {
         cx<T>* __restrict__ dst = out + v * (long)C::V + (long)(C::R * rd * C::PR + h) * C::PLANE;
         for (int l = tid; l < planes(rd) * C::N2; l += C::NT) {
             const int s = l / C::N2;
             const int z = l - s * C::N2;
+            cx<T>* t0 = sm + s * C::SS + z;
             cx<T> t[C::N1];
 #pragma unroll
-            for (int j = 0; j < C::N1; ++j) t[j] = sm[s * C::SS + j * C::YS + z];
+            for (int j = 0; j < C::N1; ++j) t[j] = t0[j * C::YS];
             dft<C::N1, C::S, T, C::ALG>(t, bk);
             cx<T>* __restrict__ o = dst + s * (C::R * C::PLANE) + z;
             // Always scaled: a product by 1 is exact.
 #pragma unroll
-            for (int k = 0; k < C::N1; ++k) st_hint<C::HS>(o + k * C::N2, scale(t[k], scl));
+            for (int k = 0; k < C::N1; ++k) {
+                if constexpr (C::LIN) t0[k * C::YS] = scale(t[k], scl);
+                else st_hint<C::HS>(o + k * C::N2, scale(t[k], scl));
+            }
+        }
+    }
+    // LIN = 1: the round's planes LDS -> HBM, 16 bytes a lane and consecutive lanes adjacent.
+    template <int rd>
+    static FX_HD void copy(int tid, long v, int h, const cx<T>* sm, cx<T>* __restrict__ out)
+    {
+        constexpr int W = 16 / (int)sizeof(cx<T>);   // elements per lane
+        static_assert(C::N2 % W == 0, "a lane's elements lie in one row");
+        cx<T>* __restrict__ dst = out + v * (long)C::V + (long)(C::R * rd * C::PR + h) * C::PLANE;
+#pragma unroll 4
+        for (int e = tid; e < planes(rd) * C::PLANE / W; e += C::NT) {
+            const int s = e / (C::PLANE / W);
+            const int q = (e - s * (C::PLANE / W)) * W;
+            const int y = q / C::N2;
+            const cx<T>* t = sm + s * C::SS + y * C::YS + (q - y * C::N2);
+            st_wide<C::HS>(dst + s * (C::R * C::PLANE) + q, t);
         }
     }
 };
@@ -199,6 +232,10 @@ __device__ __forceinline__ void xhold_rounds(int tid, long v, int h, const typen
     K::template zpass<rd>(tid, sm, bk);
     __syncthreads();
     K::template ypass<rd>(tid, v, h, sm, out, bk, scl);
+    if constexpr (C::LIN) {
+        __syncthreads();
+        K::template copy<rd>(tid, v, h, sm, out);
+    }
     if constexpr (rd + 1 < C::RD) xhold_rounds<C, rd + 1>(tid, v, h, H, sm, out, bk, scl);
 }
 

@@ -18,6 +18,7 @@ void emu_xhold_round(long v, int h, std::vector<Box>& H, EmuLds<typename C::T>& 
     }
     emu_threads(C::NT, [&](int t) { K::template zpass<rd>(t, sm, bk); });
     emu_threads(C::NT, [&](int t) { K::template ypass<rd>(t, v, h, sm, dst, bk, scl); });
+    if constexpr (C::LIN) emu_threads(C::NT, [&](int t) { K::template copy<rd>(t, v, h, sm, dst); });
     if (!lds.guards_ok() && g_emu_bad_block < 0) g_emu_bad_block = v;
     if constexpr (rd + 1 < C::RD) emu_xhold_round<C, rd + 1>(v, h, H, lds, dst, bk, scl);
 }
