@@ -16,6 +16,9 @@ hipError_t launch_xhold(const void* in, void* out, long nvol, const void* bank, 
     return hipGetLastError();
 }
 
+// Compute units that launch_rounds (xrounds.hpp) plans for.
+inline int rounds_cus() { return cu_count(); }
+
 template <class C>
 KernelDesc xhold_desc(const char* name)
 {

@@ -7,6 +7,7 @@
 #include "kernels.hpp"
 #include "xhold.hpp"
 #include "xres.hpp"
+#include "xrounds.hpp"
 
 namespace fx {
 
@@ -67,6 +68,41 @@ namespace fx {
     FX_XHL(N0, N1, N2, T, +1, R, NT, PR, GS, PF,                                                 \
            "xres_" #N0 "x" #N1 "x" #N2 "_" TAG "_bwd_v1r" #R "t" #NT "h" #PR "l")
 
+// Launches by rounds (xrounds.hpp): forms with R descending, the last one for full rounds.
+#define FX_R_BOTH(N0, N1, N2, TAG, FORMS)                                                        \
+    r.push_back(rounds_desc<FORMS(-1)>("xres_" #N0 "x" #N1 "x" #N2 "_" TAG "_fwd_v1rounds"));    \
+    r.push_back(rounds_desc<FORMS(+1)>("xres_" #N0 "x" #N1 "x" #N2 "_" TAG "_bwd_v1rounds"))
+#define FX_R36D(S)                                                                               \
+    ResForm<XResCfg<36, 36, 36, double, S, 12, 256, 1, 4>, 1>,                                   \
+        ResForm<XResCfg<36, 36, 36, double, S, 6, 512, 2, 4>, 1>,                                \
+        HoldForm<XHoldCfg<36, 36, 36, double, S, 4, 448, 6, 9, 2>, 1>,                           \
+        HoldForm<XHoldCfg<36, 36, 36, double, S, 2, 256, 6, 9, 3>, 1>
+#define FX_R48D(S)                                                                               \
+    ResForm<XResCfg<24, 24, 48, double, S, 8, 256, 1, 4>, 1>,                                    \
+        ResForm<XResCfg<24, 24, 48, double, S, 4, 384, 1, 2>, 1>,                                \
+        HoldForm<XHoldCfg<24, 24, 48, double, S, 2, 256, 8, 6, 4>, 1>
+#define FX_R24D(S)                                                                               \
+    ResForm<XResCfg<24, 24, 24, double, S, 6, 192, 0, 4>, 1>,                                    \
+        ResForm<XResCfg<24, 24, 24, double, S, 4, 192, 0, 4>, 1>,                                \
+        ResForm<XResCfg<24, 24, 24, double, S, 3, 256, 1, 3>, 2>
+#define FX_R36F(S)                                                                               \
+    ResForm<XResCfg<36, 36, 36, float, S, 12, 256, 1, 4>, 1>,                                    \
+        ResForm<XResCfg<36, 36, 36, float, S, 6, 448, 2, 4>, 1>,                                 \
+        ResForm<XResCfg<36, 36, 36, float, S, 3, 512, 2, 2>, 1>,                                 \
+        HoldForm<XHoldCfg<36, 36, 36, float, S, 2, 448, 9, 9, 3, 1>, 1>,                         \
+        HoldForm<XHoldCfg<36, 36, 36, float, S, 1, 448, 12, 9, 4, 1>, 1>
+#define FX_R48F(S)                                                                               \
+    ResForm<XResCfg<24, 24, 48, float, S, 6, 192, 0, 4>, 1>,                                     \
+        ResForm<XResCfg<24, 24, 48, float, S, 3, 256, 0, 3>, 1>,                                 \
+        ResForm<XResCfg<24, 24, 48, float, S, 2, 384, 0, 3>, 1>,                                 \
+        HoldForm<XHoldCfg<24, 24, 48, float, S, 1, 384, 12, 6, 4>, 1>
+#define FX_R24F(S)                                                                               \
+    ResForm<XResCfg<24, 24, 24, float, S, 6, 192, 0, 6>, 1>,                                     \
+        ResForm<XResCfg<24, 24, 24, float, S, 3, 192, 0, 4>, 1>,                                 \
+        ResForm<XResCfg<24, 24, 24, float, S, 2, 320, 0, 2>, 1>,                                 \
+        HoldForm<XHoldCfg<24, 24, 24, float, S, 1, 192, 8, 6, 4>, 2>,                            \
+        HoldForm<XHoldCfg<24, 24, 24, float, S, 1, 192, 8, 6, 4, 1>, 4>
+
 // (Pass B with plain stores, PencilCfg XH = 1, measured 8% slower at 36^3 x 128 and 1% at
 // 24x24x48 x 64 than with nontemporal ones: not registered.)
 
@@ -122,6 +158,21 @@ void register_pencil(std::vector<KernelDesc>& r)
     // pass was pipelined, xres.hpp; since then 24x24x48 x 64 takes 16.4 us with rotated blocks
     // (o1) and 16.7 with offset starts, and 24^3 x 8 6.0 us in six workgroups (r6) against 6.6
     // in four, which is the better one from x 64 on.)
+    // By rounds, ahead of the single forms so that a plan that ties takes the launch that also
+    // fits its smaller executes (single form -> by rounds, us):
+    //   36^3              x 1 27.7 -> 11.3, x 64 34.2 -> 26.4, x 150 70.0 -> 57.0, x 258 107 -> 92
+    //   24x24x48          x 1 16.5 -> 8.6, x 64 20.5 -> 16.3, x 150 42.8 -> 35.4
+    //   36^3 complex64    x 1 27.1 -> 10.4, x 64 30.8 -> 19.4, x 300 68.3 -> 56.7
+    //   24x24x48 complex64 x 1 15.4 -> 7.9, x 128 18.4 -> 14.9, x 300 40.4 -> 35.9
+    //   24^3 complex64    x 1 9.2 (LDS-resident) -> 5.0, x 85 10.3 -> 8.0, x 1024 53.4 -> 44.0
+    // 24^3 complex128 ends in r3: r2h8 is 3% faster at x 256 and 5% at x 192, and 11% slower
+    // at x 400.
+    FX_R_BOTH(36, 36, 36, "c128", FX_R36D);
+    FX_R_BOTH(24, 24, 48, "c128", FX_R48D);
+    FX_R_BOTH(24, 24, 24, "c128", FX_R24D);
+    FX_R_BOTH(36, 36, 36, "c64", FX_R36F);
+    FX_R_BOTH(24, 24, 48, "c64", FX_R48F);
+    FX_R_BOTH(24, 24, 24, "c64", FX_R24F);
     FX_XO_BOTH(36, 36, 36, double, "c128", 6, 512, 2, 4);
     FX_XO_BOTH(36, 36, 36, double, "c128", 6, 512, 1, 4);
     FX_X_BOTH(36, 36, 36, double, "c128", 6, 512, 4);

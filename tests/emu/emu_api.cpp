@@ -10,9 +10,12 @@
 namespace fx {
 int g_emu_reverse = 0;
 long g_emu_bad_block = -1;
+int g_emu_cus = 32;   // 4 per XCD: 16 volumes a round at two workgroups a volume
 }  // namespace fx
 
 using namespace fx;
+
+extern "C" void emu_set_cus(int n) { g_emu_cus = n; }
 
 extern "C" int emu_kernel_count(void) { return (int)registry().size(); }
 

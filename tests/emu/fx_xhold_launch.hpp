@@ -51,6 +51,10 @@ hipError_t launch_xhold(const void* in, void* out, long nvol, const void* bank, 
     return hipSuccess;
 }
 
+// Compute units that launch_rounds (xrounds.hpp) plans for; tests set it.
+extern int g_emu_cus;
+inline int rounds_cus() { return g_emu_cus; }
+
 template <class C>
 KernelDesc xhold_desc(const char* name)
 {
