@@ -98,44 +98,77 @@ static std::string wisdom_key(int n0, int n1, int n2, int prec, int dir, long ba
     return buf;
 }
 
-// Time one candidate: 2 warm launches, one group of 5 to size the groups, then the best of
-// 3 groups of n launches, n chosen so a group lasts about 300 us (5..64): event timing
-// jitter of a few microseconds would otherwise decide between kernels of ~10 us.
-// Successive launches use successive windows of the race buffers, so with enough windows
-// no launch finds its data in the 256 MB Infinity Cache and the race ranks kernels as they
-// run from HBM.  Seconds per launch, or -1 if it failed to launch.
-static double trial(const KernelDesc& k, const char* din, char* dout, size_t wbytes, int nwin,
-                    long nvol, const void* bank, unsigned* work, hipStream_t s, hipEvent_t e0,
-                    hipEvent_t e1)
-{
+// One candidate of a race: launches in groups of n between two events, n chosen so that a group
+// lasts about 300 us (5..64): event timing jitter of a few microseconds would otherwise decide
+// between kernels of ~10 us.  Successive launches use successive windows of the race buffers,
+// so with enough windows no launch finds its data in the 256 MB Infinity Cache and the race
+// ranks kernels as they run from HBM.
+struct Trial {
+    const KernelDesc* k;
+    int n;        // launches per group; 0: failed to launch, or out of the race
+    double best;  // fastest group, seconds per launch
+};
+
+struct RaceRig {
+    const char* din;
+    char* dout;
+    size_t wbytes;
+    int nwin;
+    long nvol;
+    const void* bank;
+    unsigned* work;
+    hipStream_t s;
+    hipEvent_t e0, e1;
     int w = 0;
-    auto launch = [&]() {
+
+    bool launch(const KernelDesc& k)
+    {
         const size_t off = (size_t)(w++ % nwin) * wbytes;
-        return k.launch(din + off, dout + off, nvol, bank, 1.0, work, s);
-    };
-    for (int i = 0; i < 2; ++i)
-        if (launch() != hipSuccess) return -1.0;
-    auto group = [&](int n) -> double {
+        return k.launch(din + off, dout + off, nvol, bank, 1.0, work, s) == hipSuccess;
+    }
+    // Seconds per launch of n launches, or -1 if one failed.
+    double group(const KernelDesc& k, int n)
+    {
         if (hipEventRecord(e0, s) != hipSuccess) return -1.0;
         for (int i = 0; i < n; ++i)
-            if (launch() != hipSuccess) return -1.0;
+            if (!launch(k)) return -1.0;
         if (hipEventRecord(e1, s) != hipSuccess) return -1.0;
         if (hipEventSynchronize(e1) != hipSuccess) return -1.0;
         float ms = 0.f;
         if (hipEventElapsedTime(&ms, e0, e1) != hipSuccess) return -1.0;
         return (double)ms * 1e-3 / n;
-    };
-    const double first = group(5);
-    if (first <= 0) return -1.0;
-    int n = (int)(300e-6 / first);
-    n = n < 5 ? 5 : (n > 64 ? 64 : n);
-    double best = 1e30;
-    for (int g = 0; g < 3; ++g) {
-        const double per = group(n);
-        if (per <= 0) return -1.0;
-        if (per < best) best = per;
     }
-    return best;
+};
+
+// Sizes every candidate's groups (which also brings the clocks up), then times the candidates
+// in turn, one group each a round, so that none has the cold or the busy end of the race to
+// itself: timed one after the other, kernels 5% apart changed places from run to run.
+// Candidates far behind drop out after the first rounds, which keeps a race of five rounds as
+// long as one of three groups each was.
+static void run_trials(RaceRig& r, std::vector<Trial>& ts)
+{
+    for (Trial& t : ts) {
+        t.n = 0;
+        t.best = 1e30;
+        if (!r.launch(*t.k) || !r.launch(*t.k)) continue;
+        const double first = r.group(*t.k, 5);
+        if (first <= 0) continue;
+        const int n = (int)(300e-6 / first);
+        t.n = n < 5 ? 5 : (n > 64 ? 64 : n);
+    }
+    const double keep[5] = {1.25, 1.12, 1.08, 1.08, 1.08};
+    for (int round = 0; round < 5; ++round) {
+        double lead = 1e30;
+        for (Trial& t : ts) {
+            if (!t.n) continue;
+            const double per = r.group(*t.k, t.n);
+            if (per <= 0) t.n = 0, t.best = 1e30;
+            else if (per < t.best) t.best = per;
+            if (t.best < lead) lead = t.best;
+        }
+        for (Trial& t : ts)
+            if (t.best > keep[round] * lead) t.n = 0;
+    }
 }
 
 // *best_s = 0 when no trial completed (no race buffers, or every launch failed): the
@@ -176,17 +209,18 @@ static const KernelDesc* race(const std::vector<const KernelDesc*>& cands, int n
     if (hipStreamCreate(&s) == hipSuccess) {
         if (hipEventCreate(&e0) == hipSuccess) {
             if (hipEventCreate(&e1) == hipSuccess) {
+                RaceRig rig{(const char*)din, (char*)dout, wbytes, nwin, rb, bank, work, s, e0, e1};
+                std::vector<Trial> ts;
+                for (const KernelDesc* k : cands) ts.push_back(Trial{k, 0, 1e30});
+                run_trials(rig, ts);
                 // A later candidate must beat the incumbent by more than 2% (about the
                 // run-to-run spread of one trial), so near-ties resolve the same way each
                 // time, to the earlier-registered variant.
-                for (const KernelDesc* k : cands) {
-                    const double t = trial(*k, (const char*)din, (char*)dout, wbytes, nwin,
-                                           rb, bank, work, s, e0, e1);
-                    if (t > 0 && (wt > 1e29 || t < 0.98 * wt)) {
-                        wt = t;
-                        win = k;
+                for (const Trial& t : ts)
+                    if (t.best < 1e29 && (wt > 1e29 || t.best < 0.98 * wt)) {
+                        wt = t.best;
+                        win = t.k;
                     }
-                }
                 (void)hipEventDestroy(e1);
             }
             (void)hipEventDestroy(e0);
