@@ -120,7 +120,8 @@ int fft3d_mx_kernel_count(void);
 const char *fft3d_mx_kernel_name(int i, int *n0, int *n1, int *n2, int *precision,
                                  int *direction);
 
-/* The plan-time constant bank, exactly as uploaded to the device, for inspection.  Layout
+/* The plan-time constant bank, exactly as uploaded to the device, for inspection (plans of the
+ * matrix-core kernels upload their matrix fragments behind it).  Layout
  * (element type double for FFT3D_MX_C128, float for FFT3D_MX_C64, complex = {re, im}):
  *   W tables, complex, concatenated for N = 2,3,4,6,8,9,12,16,17,24,36,48 (185 entries),
  *     entry m of table N = exp(-2 pi i m / N);

@@ -21,7 +21,7 @@
 // with SPLIT = 1 every line is multiplied, before the split, by the power of two that brings
 // its largest magnitude into [0.5, 1) (a maximum over the four lanes holding the line,
 // through two lane-swap moves), and its outputs by the inverse power; both scalings are
-// exact.  The matrix fragments come from the plan-time bank, are built once per workgroup
+// exact.  The matrix fragments are made at plan time (mfma_frag.hpp), loaded once per workgroup
 // and stay in VGPRs.  17-point lines may instead take the conjugate-pair fold (Fold17Matrix
 // below).
 //
@@ -36,6 +36,7 @@
 #include <type_traits>
 
 #include "kernels.hpp"
+#include "mfma_frag.hpp"
 
 namespace fx {
 
@@ -71,19 +72,13 @@ __device__ __forceinline__ V pack_words(const unsigned (&w)[NW])
     else return __builtin_bit_cast(V, mf_v4u{w[0], w[1], w[2], w[3]});
 }
 
-// Split and product for SPLIT (0 bf16, 1 fp16) and the instruction's K width.
+// Operand type and product for SPLIT (0 bf16, 1 fp16) and the instruction's K width.
 template <int SPLIT, int KW>
 struct MfmaOps;
 template <>
 struct MfmaOps<0, 16> {
     using V = mf_v4s;
     static constexpr int Q = 4;
-    __device__ __forceinline__ static void split(float x, V& hi, V& lo, int q)
-    {
-        const __bf16 h = (__bf16)x;
-        hi[q] = __builtin_bit_cast(short, h);
-        lo[q] = __builtin_bit_cast(short, (__bf16)(x - (float)h));
-    }
     __device__ __forceinline__ static mf_v4f mma(V a, V b, mf_v4f c)
     {
         return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
@@ -93,12 +88,6 @@ template <>
 struct MfmaOps<1, 16> {
     using V = mf_v4h;
     static constexpr int Q = 4;
-    __device__ __forceinline__ static void split(float x, V& hi, V& lo, int q)
-    {
-        const _Float16 h = (_Float16)x;
-        hi[q] = h;
-        lo[q] = (_Float16)(x - (float)h);
-    }
     __device__ __forceinline__ static mf_v4f mma(V a, V b, mf_v4f c)
     {
         return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
@@ -108,12 +97,6 @@ template <>
 struct MfmaOps<0, 32> {
     using V = mf_v8b;
     static constexpr int Q = 8;
-    __device__ __forceinline__ static void split(float x, V& hi, V& lo, int q)
-    {
-        const __bf16 h = (__bf16)x;
-        hi[q] = h;
-        lo[q] = (__bf16)(x - (float)h);
-    }
     __device__ __forceinline__ static mf_v4f mma(V a, V b, mf_v4f c)
     {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -123,12 +106,6 @@ template <>
 struct MfmaOps<1, 32> {
     using V = mf_v8h;
     static constexpr int Q = 8;
-    __device__ __forceinline__ static void split(float x, V& hi, V& lo, int q)
-    {
-        const _Float16 h = (_Float16)x;
-        hi[q] = h;
-        lo[q] = (_Float16)(x - (float)h);
-    }
     __device__ __forceinline__ static mf_v4f mma(V a, V b, mf_v4f c)
     {
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
@@ -179,27 +156,19 @@ struct MfmaMatrix {
     static constexpr int Q = Ops::Q;
     typename Ops::V hi[TM][TK], lo[TM][TK];
 
-    // A[m][k] of the real block matrix, rows and columns interleaved (re, im) per point.
-    __device__ __forceinline__ static float entry(int m, int k, const Bank<float>* __restrict__ bk)
-    {
-        const int o = m >> 1, j = k >> 1;
-        if (o >= N || j >= N) return 0.f;
-        const cx<float> w = bk->w[woff(N) + (o * j) % N];
-        const float wr = w.r, wi = S < 0 ? w.i : -w.i;
-        if ((m & 1) == 0) return (k & 1) == 0 ? wr : -wi;
-        return (k & 1) == 0 ? wi : wr;
-    }
     __device__ __forceinline__ void build(int lane, const Bank<float>* __restrict__ bk)
     {
+        constexpr int off = frag_set(S, SPLIT) + frag_off(N, KW, 0);
+        static_assert(frag_off(N, KW, 0) < kFragSet, "a form of kFragForms");
+        const auto* __restrict__ p =
+            reinterpret_cast<const typename Ops::V*>(reinterpret_cast<const char*>(bk) + off) + lane;
 #pragma unroll
         for (int mt = 0; mt < TM; ++mt)
 #pragma unroll
-            for (int kt = 0; kt < TK; ++kt)
-#pragma unroll
-                for (int q = 0; q < Q; ++q) {
-                    const float a = entry(16 * mt + lane % 16, KW * kt + Q * (lane / 16) + q, bk);
-                    Ops::split(a, hi[mt][kt], lo[mt][kt], q);
-                }
+            for (int kt = 0; kt < TK; ++kt) {
+                hi[mt][kt] = p[128 * (mt * TK + kt)];
+                lo[mt][kt] = p[128 * (mt * TK + kt) + 64];
+            }
     }
 };
 
@@ -220,26 +189,15 @@ struct Fold17Matrix {
     using Ops = MfmaOps<SPLIT, 32>;
     typename Ops::V ph, pl, mh, ml;   // P and M, high and low parts
 
-    // Row m (output point m/2 + 1, re/im), column c (a or b of point (c % 16)/2 + 1, re/im).
-    __device__ __forceinline__ static float entry(int m, int c, bool minus,
-                                                  const Bank<float>* __restrict__ bk)
-    {
-        const int k = m / 2 + 1, j = (c % 16) / 2 + 1;
-        const cx<float> w = bk->w[woff(17) + (j * k) % 17];   // exp(-2 pi i jk/17)
-        const float cs = w.r, sn = (S < 0 ? w.i : -w.i) * (minus ? -1.f : 1.f);   // S sin
-        const bool re_out = (m & 1) == 0, re_in = (c & 1) == 0;
-        if (c < 16) return re_out == re_in ? cs : 0.f;          // a_j c
-        if (re_out) return re_in ? 0.f : -sn;                    // Re(i b s) = -Im(b) s
-        return re_in ? sn : 0.f;                                 // Im(i b s) =  Re(b) s
-    }
     __device__ __forceinline__ void build(int lane, const Bank<float>* __restrict__ bk)
     {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const int m = lane % 16, c = 8 * (lane / 16) + q;
-            Ops::split(entry(m, c, false, bk), ph, pl, q);
-            Ops::split(entry(m, c, true, bk), mh, ml, q);
-        }
+        constexpr int off = frag_set(S, SPLIT) + frag_off(17, 32, 1);
+        const auto* __restrict__ p =
+            reinterpret_cast<const typename Ops::V*>(reinterpret_cast<const char*>(bk) + off) + lane;
+        ph = p[0];
+        pl = p[64];
+        mh = p[128];
+        ml = p[192];
     }
 };
 

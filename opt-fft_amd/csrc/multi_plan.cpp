@@ -191,8 +191,9 @@ extern "C" fft3d_mx_multi* fft3d_mx_multi_create(const fft3d_mx_item* items, int
         m->scale[i] = (flags & FFT3D_MX_NORMALIZE) ? 1.0 / ((double)it.n0 * it.n1 * it.n2) : 1.0;
     }
     if (hipGetDevice(&m->device) != hipSuccess) m->device = 0;
+    const int algo = (flags & FFT3D_MX_MFMA_BF16) ? 1 : (flags & FFT3D_MX_MFMA_FP16) ? 2 : 0;
     std::vector<unsigned char> img;
-    bank_host_image(precision, img);
+    bank_device_image(precision, algo, img);
     hipError_t e = hipMalloc(&m->bank, img.size());
     if (e == hipSuccess) e = hipMemcpy(m->bank, img.data(), img.size(), hipMemcpyHostToDevice);
     const size_t work_bytes = ClaimSlots::bytes();
@@ -206,7 +207,6 @@ extern "C" fft3d_mx_multi* fft3d_mx_multi_create(const fft3d_mx_item* items, int
         return nullptr;
     }
     m->claims.attach(m->work);
-    const int algo = (flags & FFT3D_MX_MFMA_BF16) ? 1 : (flags & FFT3D_MX_MFMA_FP16) ? 2 : 0;
     std::vector<const MultiDesc*> cands;
     const char* forced = getenv("FFT3D_MX_MULTI_KERNEL");
     for (const MultiDesc& d : multi_registry())

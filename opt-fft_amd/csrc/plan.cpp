@@ -383,7 +383,7 @@ static fft3d_mx_plan* create_impl(int n0, int n1, int n2, int batch, int directi
         p->cus = 1;
 
     std::vector<unsigned char> img;
-    bank_host_image(precision, img);
+    bank_device_image(precision, pick ? pick->algo : algo, img);
     hipError_t e = hipMalloc(&p->bank, img.size());
     if (e != hipSuccess) {
         fail(FFT3D_MX_ENOMEM, "fft3d_mx_create: hipMalloc(bank): %s", hipGetErrorString(e));

@@ -18,5 +18,8 @@ inline bool elem_aligned(const void* p, int prec)
     return (uintptr_t)p % elem_bytes(prec) == 0;
 }
 void bank_host_image(int prec, std::vector<unsigned char>& img);
+// What a plan uploads: the bank, and for kernels of algo != 0 (KernelDesc::algo) the matrix
+// fragments behind it (mfma_frag.hpp).
+void bank_device_image(int prec, int algo, std::vector<unsigned char>& img);
 
 }  // namespace fx

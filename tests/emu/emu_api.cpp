@@ -3,6 +3,7 @@
 #include <vector>
 
 #include "cx.hpp"
+#include "mfma_frag.hpp"
 #include "plan_internal.hpp"
 #include "registry.hpp"
 #include "multi_tasks.hpp"
@@ -14,6 +15,21 @@ int g_emu_cus = 32;   // 4 per XCD: 16 volumes a round at two workgroups a volum
 }  // namespace fx
 
 using namespace fx;
+
+// The matrix fragments of a complex64 matrix-core plan: bytes of set (S, split), form k.
+extern "C" int emu_frag(int S, int split, int k, int* n, int* kw, int* fold, void* dst, size_t cap)
+{
+    if (k < 0 || k >= kNumFragForms) return -1;
+    const FragForm f = kFragForms[k];
+    *n = f.n;
+    *kw = f.kw;
+    *fold = f.fold;
+    std::vector<unsigned char> img;
+    bank_device_image(kC64, 1 + split, img);
+    if ((size_t)frag_bytes(f) > cap || img.size() != (size_t)kFragEnd) return -2;
+    memcpy(dst, img.data() + frag_set(S, split) + frag_off(f.n, f.kw, f.fold), frag_bytes(f));
+    return frag_bytes(f);
+}
 
 extern "C" void emu_set_cus(int n) { g_emu_cus = n; }
 
