@@ -111,6 +111,8 @@ typedef struct fft3d_mx_plan_info {
     char kernel[96];     /* kernel name */
     long small_max;      /* executes of at most this many volumes use kernel_small (0: none) */
     char kernel_small[96];  /* small-batch kernel name ("" if none) */
+    /* (17^3: a raced plan of more than 32 (complex128) or 48 (complex64) volumes, on 256 CUs,
+       executes that many and fewer through plane_17x17x17_*, whatever the classes above.) */
 } fft3d_mx_plan_info;
 int fft3d_mx_plan_get_info(const fft3d_mx_plan *plan, fft3d_mx_plan_info *info);
 

@@ -1,6 +1,7 @@
 // Balanced 17^3 kernels (f17.hpp): complex128 at two workgroups per CU, complex64 at four,
-// both directions.
+// both directions; and the plane-per-workgroup kernels for small batches (plane17.hpp).
 #include "f17.hpp"
+#include "plane17.hpp"
 
 namespace fx {
 
@@ -17,6 +18,10 @@ void register_f17(std::vector<KernelDesc>& r)
     FX_B(float, "c64", +1, "bwd", 4);
     FX_B(float, "c64", -1, "fwd", 2);
     FX_B(float, "c64", +1, "bwd", 2);
+    r.push_back(plane17_desc<Plane17Cfg<double, -1>>("plane_17x17x17_c128_fwd_v1t320"));
+    r.push_back(plane17_desc<Plane17Cfg<double, +1>>("plane_17x17x17_c128_bwd_v1t320"));
+    r.push_back(plane17_desc<Plane17Cfg<float, -1>>("plane_17x17x17_c64_fwd_v1t320"));
+    r.push_back(plane17_desc<Plane17Cfg<float, +1>>("plane_17x17x17_c64_bwd_v1t320"));
 }
 
 }  // namespace fx

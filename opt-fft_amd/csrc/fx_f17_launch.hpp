@@ -10,7 +10,8 @@ hipError_t launch_f17(const void* in, void* out, long nvol, const void* bank, do
     using T = typename C::T;
     if (nvol <= 0) return hipSuccess;
     if (nvol >= (1L << 31)) return hipErrorInvalidValue;
-    const long grid = persistent_grid(k_f17<C>, C::NT, C::PERSIST, nvol);
+    static const int per = resident_per_cu(k_f17<C>, C::NT);
+    const long grid = persistent_grid(per, C::PERSIST, nvol);
     hipLaunchKernelGGL((k_f17<C>), dim3((unsigned)grid), dim3(C::NT), 0, stream,
                        (const cx<T>*)in, (cx<T>*)out, nvol, (const Bank<T>*)bank, (T)scl,
                        claim_counter(work, grid, nvol));

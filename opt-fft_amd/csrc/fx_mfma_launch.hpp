@@ -11,7 +11,8 @@ hipError_t launch_mfma(const void* in, void* out, long nvol, const void* bank, d
     const long nblocks = (nvol + C::VPW - 1) / C::VPW;
     if (nblocks >= (1L << 31)) return hipErrorInvalidValue;
     if constexpr (PERSIST > 0) {
-        const long grid = persistent_grid(k_mfma_pipe<C, SPLIT, KW, PERSIST, XD>, C::NT, PERSIST, nblocks);
+        static const int per = resident_per_cu(k_mfma_pipe<C, SPLIT, KW, PERSIST, XD>, C::NT);
+        const long grid = persistent_grid(per, PERSIST, nblocks);
         hipLaunchKernelGGL((k_mfma_pipe<C, SPLIT, KW, PERSIST, XD>), dim3((unsigned)grid), dim3(C::NT),
                            0, stream, (const cx<float>*)in, (cx<float>*)out, nvol, nblocks,
                            (const Bank<float>*)bank, (float)scl);

@@ -6,7 +6,8 @@ namespace fx {
 template <typename T, int PRESET>
 long multi_launch_grid(long ntasks)
 {
-    return persistent_grid(k_multi<T, PRESET>, MultiCfg<T, PRESET>::NT, 8, ntasks);
+    static const int per = resident_per_cu(k_multi<T, PRESET>, MultiCfg<T, PRESET>::NT);
+    return persistent_grid(per, 8, ntasks);
 }
 
 template <typename T, int PRESET>
@@ -36,7 +37,8 @@ template <typename T, int PRESET>
 int multi_dev_grid()
 {
     using M = MultiCfg<T, PRESET>;
-    return (int)persistent_grid(k_multi_dev<T, PRESET>, M::NT, 8, 1L << 30);
+    static const int per = resident_per_cu(k_multi_dev<T, PRESET>, M::NT);
+    return (int)persistent_grid(per, 8, 1L << 30);
 }
 
 template <typename T, int PRESET>

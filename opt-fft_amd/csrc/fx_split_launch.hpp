@@ -10,7 +10,11 @@ hipError_t launch_split(const void* in, void* out, long nvol, const void* bank, 
     using T = typename C::T;
     if (nvol <= 0) return hipSuccess;
     if (nvol >= (1L << 31)) return hipErrorInvalidValue;
-    const long grid = C::P > 0 ? persistent_grid(k_split<C>, C::NT, C::P, nvol) : nvol;
+    long grid = nvol;
+    if constexpr (C::P > 0) {
+        static const int per = resident_per_cu(k_split<C>, C::NT);
+        grid = persistent_grid(per, C::P, nvol);
+    }
     hipLaunchKernelGGL((k_split<C>), dim3((unsigned)grid), dim3(C::NT), 0, stream,
                        (const cx<T>*)in, (cx<T>*)out, nvol, (const Bank<T>*)bank, (T)scl,
                        C::P > 0 ? claim_counter(work, grid, nvol) : nullptr);

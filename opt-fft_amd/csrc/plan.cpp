@@ -247,6 +247,10 @@ struct fft3d_mx_plan {
     // eighth of the planned batch) when it differs from k; NULL otherwise.
     const KernelDesc* k_small;
     long small_max;
+    // Tiny class (KernelDesc::tiny): executes of at most tiny_max volumes launch k_tiny when it
+    // is not NULL (plans whose kernel was raced, at batches above tiny_max).
+    const KernelDesc* k_tiny;
+    long tiny_max;
     void* bank;
     unsigned* work;     // device: the claim counters `claims` hands out (claims.hpp)
     ClaimSlots claims;
@@ -272,6 +276,7 @@ static bool may_claim(const fft3d_mx_plan* p, const KernelDesc* k, long batch)
 // The plan's kernel for a launch of `batch` volumes.
 static const KernelDesc* kernel_for(const fft3d_mx_plan* p, long batch)
 {
+    if (p->k_tiny && batch <= p->tiny_max) return p->k_tiny;
     return p->k_small && batch <= p->small_max ? p->k_small : p->k;
 }
 
@@ -411,6 +416,8 @@ static fft3d_mx_plan* create_impl(int n0, int n1, int n2, int batch, int directi
 
     p->k_small = nullptr;
     p->small_max = 0;
+    p->k_tiny = nullptr;
+    p->tiny_max = 0;
     if (!pick) {
         if (cands.size() == 1 || (flags & FFT3D_MX_NO_TUNE) || batch == 0) {
             pick = cands[0];
@@ -440,6 +447,13 @@ static fft3d_mx_plan* create_impl(int n0, int n1, int n2, int batch, int directi
                 if (ks != pick) {
                     p->k_small = ks;
                     p->small_max = (long)std::sqrt((double)batch * (double)bs);
+                }
+            }
+            for (const KernelDesc* k : cands) {
+                const long most = (long)k->tiny * p->cus / 256;
+                if (most > 0 && batch > most) {
+                    p->k_tiny = k;
+                    p->tiny_max = most;
                 }
             }
         }

@@ -36,6 +36,9 @@ struct KernelDesc {
     const char* name;
     LaunchFn launch;
     int algo = 0;    // 0 exact FP FFT; 1 DFT matrix on MFMA, split bf16; 2 split fp16
+    // Volumes per 256 CUs up to which this kernel is the quickest of its geometry: plans whose
+    // kernel was raced launch it there, whatever won at their batch.  0: no such class.
+    int tiny = 0;
 };
 
 // Appended by each kernel translation unit.
