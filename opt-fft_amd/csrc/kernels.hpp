@@ -67,6 +67,33 @@ FX_HD void stage_full(int tid, const cx<T>* __restrict__ src, cx<T>* sm, SlotFn 
     }
 }
 
+// Small index arithmetic at full rate: 32-bit multiplies and the compiler's divisions by
+// constants (a high multiply) issue at a quarter of it, and a tile of the matrix-core kernels
+// spent as long on seven of them as on everything else.
+FX_HD unsigned mul24(unsigned a, unsigned b)   // a, b < 2^24
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __umul24(a, b);
+#else
+    return a * b;
+#endif
+}
+// l / D for 0 <= l <= MAX.
+template <int D, int MAX>
+FX_HD int quot(int l)
+{
+    if constexpr (MAX < D) {
+        return 0;
+    } else if constexpr ((D & (D - 1)) == 0) {
+        return (int)((unsigned)l / D);
+    } else {
+        // M = (2^20 + e) / D with 0 < e <= D: exact while l e < 2^20, the product in 32 bits.
+        constexpr unsigned M = (1u << 20) / D + 1;
+        static_assert(D > 1 && MAX < (1 << 20) / D && MAX < 4096 * (D - 1), "in range");
+        return (int)(mul24((unsigned)l, M) >> 20);
+    }
+}
+
 // In-LDS line pass: line l starts at base(l), its N points are STRIDE apart.
 template <int N, int STRIDE, int S, int V17, int NT, typename T, typename BaseFn>
 FX_HD void lds_pass(int tid, cx<T>* sm, int nlines, BaseFn base, const Bank<T>* __restrict__ bk)
@@ -94,9 +121,16 @@ constexpr int waves_per_eu(int lds_bytes, int nt, int cap_wgs)
 }
 
 // ------------------------------------------------------------------------------- fused
+// IX = 1: indices through quot and mul24 (Fused).  The matrix-core kernels, whose tiles are short,
+// all use it: bf16x3 mix 174.1 -> 164.5 us, fp16x3 198.5 -> 179.3 (with the integer line maximum),
+// 6^3 x 65536 fp16x3 61.2 -> 49.8.  So do the complex64 FFTs above 6^3 (12^3 x 723 6.4 -> 5.7 us,
+// 8x8x16 x 3662 13.1 -> 12.1, within 1% from 150 MB on).  Elsewhere it loses more than it gains:
+// 12^3 complex128 x 361 6.5 -> 6.0 but x 1085 11.1 -> 12.2, 6^3 complex64 x 5787 5.9 -> 5.7 but x
+// 65536 40.1 -> 40.8 and more, 6^3 complex128 x 63657 78.3 -> 80.4.
 template <int N0_, int N1_, int N2_, typename T_, int S_, int VPW_, int NT_, int PZ_, int PY_,
-          int V17_>
+          int V17_, int IX_ = (sizeof(T_) == 4 && N0_ * N1_ * N2_ > 216)>
 struct FusedCfg {
+    static constexpr int IX = IX_;
     using T = T_;
     static constexpr int N0 = N0_, N1 = N1_, N2 = N2_, S = S_, VPW = VPW_, NT = NT_;
     static constexpr int PZ = PZ_, PY = PY_, V17 = V17_;
@@ -113,7 +147,58 @@ struct FusedCfg {
 template <class C>
 struct Fused {
     using T = typename C::T;
+    static_assert(!C::IX || C::PY == 0, "rows at one pitch throughout a block: the IX sums rely on it");
 
+    // LDS index of the first point of a line: z lines l = (v, x, y), y lines (v, x, z), x lines
+    // (v, y, z), each in the order of the block's elements; and the offset of its first element
+    // in the block's HBM range.
+    static FX_HD int zline(int l)
+    {
+        if constexpr (C::IX) return (int)mul24((unsigned)l, C::YS);
+        const int v = l / (C::N0 * C::N1);
+        const int r = l - v * (C::N0 * C::N1);
+        const int x = r / C::N1;
+        const int y = r - x * C::N1;
+        return v * C::VS + x * C::XS + y * C::YS;
+    }
+    static FX_HD int yrow(int l) { return quot<C::N2, C::VPW * C::N0 * C::N2>(l); }
+    static FX_HD int yline(int l)
+    {
+        if constexpr (C::IX) return l + (int)mul24((unsigned)yrow(l), C::XS - C::N2);
+        const int v = l / (C::N0 * C::N2);
+        const int r = l - v * (C::N0 * C::N2);
+        const int x = r / C::N2;
+        const int z = r - x * C::N2;
+        return v * C::VS + x * C::XS + z;
+    }
+    static FX_HD long yfirst(int l)
+    {
+        if constexpr (C::IX) return l + (int)mul24((unsigned)yrow(l), C::PLANE - C::N2);
+        const int v = l / (C::N0 * C::N2);
+        const int r = l - v * (C::N0 * C::N2);
+        const int x = r / C::N2;
+        const int z = r - x * C::N2;
+        return (long)v * C::V + x * C::PLANE + z;
+    }
+    static FX_HD int xvol(int l) { return quot<C::PLANE, C::VPW * C::PLANE - 1>(l); }
+    static FX_HD int xline(int l)
+    {
+        if constexpr (C::IX)
+            return l + quot<C::N2, C::VPW * C::PLANE>(l) * C::PZ +
+                   (int)mul24((unsigned)xvol(l), C::VS - C::XS);
+        const int v = l / C::PLANE;
+        const int q = l - v * C::PLANE;
+        const int y = q / C::N2;
+        const int z = q - y * C::N2;
+        return v * C::VS + y * C::YS + z;
+    }
+    static FX_HD long xfirst(int l)
+    {
+        if constexpr (C::IX) return l + (int)mul24((unsigned)xvol(l), C::V - C::PLANE);
+        const int v = l / C::PLANE;
+        const int q = l - v * C::PLANE;
+        return (long)v * C::V + q;
+    }
     // Volumes held by block `bid` (VPW except for the last block).
     static FX_HD int nvols(long bid, long nvol)
     {
@@ -122,6 +207,7 @@ struct Fused {
     }
     static FX_HD int slot(int e)
     {
+        if constexpr (C::IX) return e + quot<C::N2, C::VPW * C::V>(e) * C::PZ;
         const int v = e / C::V;
         const int r = e - v * C::V;
         const int x = r / C::PLANE;
@@ -145,28 +231,14 @@ struct Fused {
     {
         lds_pass<C::N2, 1, C::S, C::V17, C::NT>(
             tid, sm, nvols(bid, nvol) * C::N0 * C::N1,
-            [](int l) {
-                const int v = l / (C::N0 * C::N1);
-                const int r = l - v * (C::N0 * C::N1);
-                const int x = r / C::N1;
-                const int y = r - x * C::N1;
-                return v * C::VS + x * C::XS + y * C::YS;
-            },
-            bk);
+            [](int l) { return zline(l); }, bk);
     }
     // Phase 3: y lines (v, x, z), stride YS.
     static FX_HD void ypass(int tid, long bid, long nvol, cx<T>* sm, const Bank<T>* __restrict__ bk)
     {
         lds_pass<C::N1, C::YS, C::S, C::V17, C::NT>(
             tid, sm, nvols(bid, nvol) * C::N0 * C::N2,
-            [](int l) {
-                const int v = l / (C::N0 * C::N2);
-                const int r = l - v * (C::N0 * C::N2);
-                const int x = r / C::N2;
-                const int z = r - x * C::N2;
-                return v * C::VS + x * C::XS + z;
-            },
-            bk);
+            [](int l) { return yline(l); }, bk);
     }
     // Phase 4: x lines (v, y, z), LDS -> HBM; a wave's stores are contiguous in (y, z).
     static FX_HD void xpass(int tid, long bid, long nvol, const cx<T>* sm, cx<T>* __restrict__ out,
@@ -176,16 +248,12 @@ struct Fused {
         cx<T>* __restrict__ dst = out + bid * C::VPW * (long)C::V;
         const bool scaled = scl != T(1);
         for (int l = tid; l < nv * C::PLANE; l += C::NT) {
-            const int v = l / C::PLANE;
-            const int q = l - v * C::PLANE;
-            const int y = q / C::N2;
-            const int z = q - y * C::N2;
-            const int b = v * C::VS + y * C::YS + z;
+            const int b = xline(l);
             cx<T> t[C::N0];
 #pragma unroll
             for (int j = 0; j < C::N0; ++j) t[j] = sm[b + j * C::XS];
             dft<C::N0, C::S, T, C::V17>(t, bk);
-            cx<T>* __restrict__ o = dst + (long)v * C::V + q;
+            cx<T>* __restrict__ o = dst + xfirst(l);
             if (scaled) {
 #pragma unroll
                 for (int k = 0; k < C::N0; ++k)
@@ -248,9 +316,7 @@ struct FusedPipe {
         for (int i = 0; i < LPT; ++i) {
             int l = tid + i * C::NT;
             l = l < nl ? l : nl - 1;
-            const int v = l / C::PLANE;
-            const int q = l - v * C::PLANE;
-            const cx<T>* __restrict__ p = src + (long)v * C::V + q;
+            const cx<T>* __restrict__ p = src + Fused<C>::xfirst(l);
 #pragma unroll
             for (int j = J0; j < J1; ++j) R[i][j] = ld_hint<C::HN & 1>(p + j * C::PLANE);
         }
@@ -264,11 +330,7 @@ struct FusedPipe {
         for (int i = 0; i < LPT; ++i) {
             const int l = tid + i * C::NT;
             if (l < nl) {
-                const int v = l / C::PLANE;
-                const int q = l - v * C::PLANE;
-                const int y = q / C::N2;
-                const int z = q - y * C::N2;
-                const int s0 = v * C::VS + y * C::YS + z;
+                const int s0 = Fused<C>::xline(l);
                 dft_put<C::N0, C::S, T, C::V17>(R[i], bk,
                                                 [&](int k, cx<T> w) { sm[s0 + k * C::XS] = w; });
             }
@@ -287,15 +349,11 @@ struct FusedPipe {
         cx<T>* __restrict__ dst = out + b * C::VPW * (long)C::V;
         const bool scaled = scl != T(1);
         for (int l = tid; l < nv * C::N0 * C::N2; l += C::NT) {
-            const int v = l / (C::N0 * C::N2);
-            const int r = l - v * (C::N0 * C::N2);
-            const int x = r / C::N2;
-            const int z = r - x * C::N2;
-            const int s0 = v * C::VS + x * C::XS + z;
+            const int s0 = Fused<C>::yline(l);
             cx<T> t[C::N1];
 #pragma unroll
             for (int j = 0; j < C::N1; ++j) t[j] = sm[s0 + j * C::YS];
-            cx<T>* __restrict__ o = dst + (long)v * C::V + x * C::PLANE + z;
+            cx<T>* __restrict__ o = dst + Fused<C>::yfirst(l);
             // Hinted only where a z run fills whole 128 B lines, so that every store
             // instruction of a wave writes complete lines; shorter runs are completed by
             // later instructions and lose with the streaming policy.

@@ -13,7 +13,7 @@
 namespace fx {
 
 #define FX_MG(N0, N1, N2, S, VPW, NT, PZ, SPLIT, KW, P, XD, NAME)                                \
-    r.push_back(mfma_desc<FusedCfg<N0, N1, N2, float, S, VPW, NT, PZ, 0, 0>, SPLIT, KW, P, XD>( \
+    r.push_back(mfma_desc<FusedCfg<N0, N1, N2, float, S, VPW, NT, PZ, 0, 0, 1>, SPLIT, KW, P, XD>( \
         NAME))
 // Both directions and both splits of one form; TAG is the form's part of the name.
 #define FX_MG4(N0, N1, N2, VPW, NT, PZ, KW, P, XD, TAG)                                         \

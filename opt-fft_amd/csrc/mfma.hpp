@@ -137,11 +137,25 @@ __device__ __forceinline__ float sum_xor16(float v)
     return v + __builtin_bit_cast(float, r[0] ^ r[1] ^ u);
 }
 
-// Largest of v over the four lanes that hold one line's operand values (l, l ^ 16, l ^ 32,
-// l ^ 48).  v >= 0, so its bit pattern orders like its value.
-__device__ __forceinline__ float line_max(float v)
+// Bits of |x|: they order like the value (a float maximum would first canonicalize each operand).
+__device__ __forceinline__ unsigned abs_bits(float x)
 {
-    return __builtin_bit_cast(float, max_xor32(max_xor16(__builtin_bit_cast(unsigned, v))));
+    return __builtin_bit_cast(unsigned, x) & 0x7FFFFFFFu;
+}
+__device__ __forceinline__ unsigned max3(unsigned a, unsigned b, unsigned c)
+{
+    const unsigned m = a > b ? a : b;
+    return m > c ? m : c;
+}
+// The powers of two that bring a line into [0.5, 1) and its outputs back, times scl.  mx: this
+// lane's largest abs_bits; the largest over the four lanes that hold the line (l, l ^ 16, l ^ 32,
+// l ^ 48) decides.  frexp's exponent of 0 is 0.
+__device__ __forceinline__ void line_scale(unsigned mx, float scl, float& up, float& down)
+{
+    const float m = __builtin_bit_cast(float, max_xor32(max_xor16(mx)));
+    const int e = __builtin_amdgcn_frexp_expf(m);
+    up = ldexpf(1.f, -e);
+    down = ldexpf(scl, e);
 }
 
 // Matrix fragments of one line length N for this lane: hi and lo parts, TM x TK tiles.
@@ -276,7 +290,7 @@ __device__ __forceinline__ void mfma_pass(const cx<float>* sm, int nlines, BaseF
         const bool valid = line < nlines;
         const int b = base(valid ? line : nlines - 1);
         float v[TK][Q];
-        float mx = 0.f;
+        unsigned mx = 0;
 #pragma unroll
         for (int kt = 0; kt < TK; ++kt)
 #pragma unroll
@@ -284,16 +298,10 @@ __device__ __forceinline__ void mfma_pass(const cx<float>* sm, int nlines, BaseF
                 const cx<float> x = sm[b + goff[kt][p]];
                 v[kt][2 * p] = x.r;
                 v[kt][2 * p + 1] = x.i;
-                mx = fmaxf(mx, fmaxf(fabsf(x.r), fabsf(x.i)));
+                mx = max3(mx, abs_bits(x.r), abs_bits(x.i));
             }
         float up = 1.f, down = scl;
-        if constexpr (SPLIT == 1) {
-            mx = line_max(mx);
-            int e = 0;
-            if (mx > 0.f) (void)frexpf(mx, &e);
-            up = ldexpf(1.f, -e);
-            down = ldexpf(scl, e);
-        }
+        if constexpr (SPLIT == 1) line_scale(mx, scl, up, down);
         typename Ops::V bh[TK], bl[TK];
 #pragma unroll
         for (int kt = 0; kt < TK; ++kt) {
@@ -345,7 +353,8 @@ __device__ __forceinline__ void mfma_pass(const cx<float>* sm, int nlines, BaseF
         const int b = base(valid ? line : nlines - 1);
         const cx<float> x0 = sm[b];
         float v[8];
-        float mx = 0.f, sr = 0.f, si = 0.f;
+        unsigned mx = 0;
+        float sr = 0.f, si = 0.f;
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
             const cx<float> u = sm[b + (j0 + p) * STRIDE];
@@ -354,19 +363,13 @@ __device__ __forceinline__ void mfma_pass(const cx<float>* sm, int nlines, BaseF
             v[2 * p + 1] = fmaf(sg, w.i, u.i);
             sr += v[2 * p];
             si += v[2 * p + 1];
-            mx = fmaxf(mx, fmaxf(fabsf(v[2 * p]), fabsf(v[2 * p + 1])));
+            mx = max3(mx, abs_bits(v[2 * p]), abs_bits(v[2 * p + 1]));
         }
         // X_0: the a sums of groups 0 and 1 (groups 2 and 3 exchange b sums, unused).
         sr = sum_xor16(sr);
         si = sum_xor16(si);
         float up = 1.f, down = scl;
-        if constexpr (SPLIT == 1) {
-            mx = line_max(mx);
-            int e = 0;
-            if (mx > 0.f) (void)frexpf(mx, &e);
-            up = ldexpf(1.f, -e);
-            down = ldexpf(scl, e);
-        }
+        if constexpr (SPLIT == 1) line_scale(mx, scl, up, down);
         unsigned wh[4], wl[4];
 #pragma unroll
         for (int p = 0; p < 4; ++p) split_pair<SPLIT>(v[2 * p] * up, v[2 * p + 1] * up, wh[p], wl[p]);
@@ -411,31 +414,21 @@ __device__ __forceinline__ void mfma_passes(long bid, long nvol, cx<float>* __re
     const int nv = Fused<C>::nvols(bid, nvol);
     mfma_pass<C::N2, 1, C::S, SPLIT, C::NT>(
         sm, nv * C::N0 * C::N1,
-        [](int l) {
-            const unsigned u = (unsigned)l, v = u / (C::N0 * C::N1), r = u - v * (C::N0 * C::N1);
-            return (int)(v * C::VS + (r / C::N1) * C::XS + (r % C::N1) * C::YS);
-        },
+        [](int l) { return Fused<C>::zline(l); },
         A.z(), 1.f, [sm](int b, int, int o, cx<float> y) { sm[b + o] = y; });
     __syncthreads();
     mfma_pass<C::N1, C::YS, C::S, SPLIT, C::NT>(
         sm, nv * C::N0 * C::N2,
-        [](int l) {
-            const unsigned u = (unsigned)l, v = u / (C::N0 * C::N2), r = u - v * (C::N0 * C::N2);
-            return (int)(v * C::VS + (r / C::N2) * C::XS + (r % C::N2));
-        },
+        [](int l) { return Fused<C>::yline(l); },
         A.y(), 1.f, [sm](int b, int, int o, cx<float> y) { sm[b + o * C::YS] = y; });
     __syncthreads();
     cx<float>* __restrict__ dst = out + bid * C::VPW * (long)C::V;
     const float ci = conj ? -1.f : 1.f;
-    auto xbase = [](int l) {
-        const unsigned u = (unsigned)l, v = u / C::PLANE, q = u - v * C::PLANE;
-        return (int)(v * C::VS + (q / C::N2) * C::YS + (q % C::N2));
-    };
+    auto xbase = [](int l) { return Fused<C>::xline(l); };
     if constexpr (XD == 1) {
         mfma_pass<C::N0, C::XS, C::S, SPLIT, C::NT>(
             sm, nv * C::PLANE, xbase, A.x(), scl, [dst, ci](int, int l, int o, cx<float> y) {
-                const unsigned u = (unsigned)l, v = u / C::PLANE;
-                st_stream(dst + (long)(u + v * (C::V - C::PLANE)) + (long)o * C::PLANE,
+                st_stream(dst + (unsigned)((int)Fused<C>::xfirst(l) + (int)mul24((unsigned)o, C::PLANE)),
                           cx<float>{y.r, ci * y.i});
             });
     } else {

@@ -12,11 +12,11 @@ namespace fx {
 // standalone kernels' best) only adds tasks: 200.8 against 192.9 us for the bf16x3 mix.
 struct MultiMfmaPreset {
     static constexpr int NT = 256;
-    using G0 = FusedCfg<6, 6, 6, float, -1, 16, NT, 1, 0, 0>;
-    using G1 = FusedCfg<8, 8, 8, float, -1, 8, NT, 1, 0, 0>;
-    using G2 = FusedCfg<12, 12, 12, float, -1, 2, NT, 1, 0, 0>;
-    using G3 = FusedCfg<17, 17, 17, float, -1, 1, NT, 0, 0, 0>;
-    using G4 = FusedCfg<8, 8, 16, float, -1, 4, NT, 1, 0, 0>;
+    using G0 = FusedCfg<6, 6, 6, float, -1, 16, NT, 1, 0, 0, 1>;
+    using G1 = FusedCfg<8, 8, 8, float, -1, 8, NT, 1, 0, 0, 1>;
+    using G2 = FusedCfg<12, 12, 12, float, -1, 2, NT, 1, 0, 0, 1>;
+    using G3 = FusedCfg<17, 17, 17, float, -1, 1, NT, 0, 0, 0, 1>;
+    using G4 = FusedCfg<8, 8, 16, float, -1, 4, NT, 1, 0, 0, 1>;
     static constexpr int LDS =
         cmax(cmax(cmax(G0::LDS, G1::LDS), cmax(G2::LDS, G3::LDS)), G4::LDS);
     static constexpr int WPE = waves_per_eu(LDS * (int)sizeof(cx<float>), NT, 0);
