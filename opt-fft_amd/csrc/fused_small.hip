@@ -37,6 +37,13 @@ namespace fx {
     FX_PV(N0, N1, N2, T, +1, VPW, NT, PZ, P, ALG,                                                 \
           "pipe_" #N0 "x" #N1 "x" #N2 "_" TAG "_bwd_v" #VPW "t" #NT "p" #P SUF)
 
+// Linear stores (FusedCfg LIN): "...l".
+#define FX_FL(N0, N1, N2, T, S, VPW, NT, PZ, NAME) \
+    r.push_back(fused_desc<FusedCfg<N0, N1, N2, T, S, VPW, NT, PZ, 0, 0, 1, 1>>(NAME))
+#define FX_FL_BOTH(N0, N1, N2, T, TAG, VPW, NT, PZ)                                         \
+    FX_FL(N0, N1, N2, T, -1, VPW, NT, PZ, "fused_" #N0 "x" #N1 "x" #N2 "_" TAG "_fwd_v" #VPW "t" #NT "l"); \
+    FX_FL(N0, N1, N2, T, +1, VPW, NT, PZ, "fused_" #N0 "x" #N1 "x" #N2 "_" TAG "_bwd_v" #VPW "t" #NT "l")
+
 #define FX_S(T, S, W, PERM, X, NAME) r.push_back(shfl8_desc<Shfl8Cfg<T, S, W, PERM, X>>(NAME))
 #define FX_S_BOTH(T, TAG, W, PERM, ORD, X, XT)                                       \
     FX_S(T, -1, W, PERM, X, "shfl_8x8x8_" TAG "_fwd_w" #W ORD XT);                   \
@@ -61,6 +68,9 @@ void register_fused_small(std::vector<KernelDesc>& r)
     FX_P_BOTH(6, 6, 6, float, "c64", 16, 576, 1, 0);
     FX_F_BOTH(6, 6, 6, float, "c64", 16, 576, 1);
     FX_F_BOTH(6, 6, 6, float, "c64", 4, 144, 1);
+    FX_FL_BOTH(6, 6, 6, double, "c128", 4, 144, 1);
+    FX_FL_BOTH(6, 6, 6, float, "c64", 4, 144, 1);
+    FX_FL_BOTH(6, 6, 6, float, "c64", 8, 288, 1);
     // L = 8: 64 lines per volume per pass.
     // 8 volumes x 512 threads first: the fastest from HBM at batch 4096 (the race keeps the
     // earlier-registered variant on near-ties).

@@ -32,6 +32,8 @@
 // phases are plain __host__ __device__ functions of (thread, block).  Launchers come from
 // <fx_launch.hpp>, found on the include path.
 #pragma once
+#include <stdint.h>
+
 #include "claim_layout.hpp"
 #include "codelets.hpp"
 #include "registry.hpp"
@@ -127,10 +129,16 @@ constexpr int waves_per_eu(int lds_bytes, int nt, int cap_wgs)
 // 8x8x16 x 3662 13.1 -> 12.1, within 1% from 150 MB on).  Elsewhere it loses more than it gains:
 // 12^3 complex128 x 361 6.5 -> 6.0 but x 1085 11.1 -> 12.2, 6^3 complex64 x 5787 5.9 -> 5.7 but x
 // 65536 40.1 -> 40.8 and more, 6^3 complex128 x 63657 78.3 -> 80.4.
+//
+// LIN = 1: the last pass leaves its lines in LDS and a copy stores the block, 16 bytes a lane in
+// whole 128-byte lines, where the pass's own runs (a plane's 36 elements at 6^3, a row's 17) are
+// not: 6^3 x 65536 complex64 39.6 -> 37.4 us, 6^3 x 32768 complex128 40.7 -> 37.9, 17^3 x 2048
+// complex64 37.4 -> 36.5.  At 8^3 and 12^3, whose planes are whole lines, it is within 1%
+// (complex64) or slower (complex128: 12^3 x 4096 39.0 -> 40.0, 8^3 x 4096 10.8 -> 11.4).
 template <int N0_, int N1_, int N2_, typename T_, int S_, int VPW_, int NT_, int PZ_, int PY_,
-          int V17_, int IX_ = (sizeof(T_) == 4 && N0_ * N1_ * N2_ > 216)>
+          int V17_, int IX_ = (sizeof(T_) == 4 && N0_ * N1_ * N2_ > 216), int LIN_ = 0>
 struct FusedCfg {
-    static constexpr int IX = IX_;
+    static constexpr int IX = IX_, LIN = LIN_;
     using T = T_;
     static constexpr int N0 = N0_, N1 = N1_, N2 = N2_, S = S_, VPW = VPW_, NT = NT_;
     static constexpr int PZ = PZ_, PY = PY_, V17 = V17_;
@@ -240,11 +248,41 @@ struct Fused {
             tid, sm, nvols(bid, nvol) * C::N0 * C::N2,
             [](int l) { return yline(l); }, bk);
     }
+    // LIN = 1, after the last pass left its lines in LDS: block LDS -> HBM, 16 bytes a lane from
+    // the block's first 128-byte boundary on.
+    static FX_HD void copy(int tid, long bid, long nvol, const cx<T>* sm, cx<T>* __restrict__ out)
+    {
+        constexpr int W = 16 / (int)sizeof(cx<T>), LINE = 128 / (int)sizeof(cx<T>);
+        const int n = nvols(bid, nvol) * C::V;
+        cx<T>* __restrict__ dst = out + bid * C::VPW * (long)C::V;
+        const int head = (int)(((uintptr_t)dst / sizeof(cx<T>)) % LINE);   // elements into its line
+        for (int e = tid * W - head; e < n; e += C::NT * W) {
+            if (e >= 0 && e + W <= n) {
+                cx<T> t[W];
+#pragma unroll
+                for (int i = 0; i < W; ++i) t[i] = sm[slot(e + i)];
+                st_wide<1>(dst + e, t);
+            } else {
+                for (int i = e < 0 ? 0 : e; i < (e + W < n ? e + W : n); ++i) st_hint<1>(dst + i, sm[slot(i)]);
+            }
+        }
+    }
     // Phase 4: x lines (v, y, z), LDS -> HBM; a wave's stores are contiguous in (y, z).
-    static FX_HD void xpass(int tid, long bid, long nvol, const cx<T>* sm, cx<T>* __restrict__ out,
+    static FX_HD void xpass(int tid, long bid, long nvol, cx<T>* sm, cx<T>* __restrict__ out,
                             const Bank<T>* __restrict__ bk, T scl)
     {
         const int nv = nvols(bid, nvol);
+        if constexpr (C::LIN) {
+            for (int l = tid; l < nv * C::PLANE; l += C::NT) {
+                const int b = xline(l);
+                cx<T> t[C::N0];
+#pragma unroll
+                for (int j = 0; j < C::N0; ++j) t[j] = sm[b + j * C::XS];
+                dft_put<C::N0, C::S, T, C::V17>(
+                    t, bk, [&](int k, cx<T> w) { sm[b + k * C::XS] = scale(w, scl); });
+            }
+            return;
+        }
         cx<T>* __restrict__ dst = out + bid * C::VPW * (long)C::V;
         const bool scaled = scl != T(1);
         for (int l = tid; l < nv * C::PLANE; l += C::NT) {
@@ -282,6 +320,10 @@ __global__ void __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::W
     K::ypass(tid, bid, nvol, sm, bk);
     __syncthreads();
     K::xpass(tid, bid, nvol, sm, out, bk, scl);
+    if constexpr (C::LIN) {
+        __syncthreads();
+        K::copy(tid, bid, nvol, sm, out);
+    }
 }
 
 // ---------------------------------------------------------------------- fused, pipelined
@@ -342,10 +384,23 @@ struct FusedPipe {
     }
     // y lines (v, x, z): LDS -> HBM.
     // cj: conjugate every output (the backward transform through the forward path).
-    static FX_HD void ypass(int tid, long b, long nvol, const cx<T>* sm, cx<T>* __restrict__ out,
+    static FX_HD void ypass(int tid, long b, long nvol, cx<T>* sm, cx<T>* __restrict__ out,
                             const Bank<T>* __restrict__ bk, T scl, bool cj = false)
     {
         const int nv = nvols(b, nvol);
+        if constexpr (C::LIN) {
+            for (int l = tid; l < nv * C::N0 * C::N2; l += C::NT) {
+                const int s0 = Fused<C>::yline(l);
+                cx<T> t[C::N1];
+#pragma unroll
+                for (int j = 0; j < C::N1; ++j) t[j] = sm[s0 + j * C::YS];
+                const T si = cj ? -scl : scl;
+                dft_put<C::N1, C::S, T, C::V17>(t, bk, [&](int k, cx<T> w) {
+                    sm[s0 + k * C::YS] = cx<T>{w.r * scl, w.i * si};
+                });
+            }
+            return;
+        }
         cx<T>* __restrict__ dst = out + b * C::VPW * (long)C::V;
         const bool scaled = scl != T(1);
         for (int l = tid; l < nv * C::N0 * C::N2; l += C::NT) {
@@ -483,6 +538,10 @@ __global__ void __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::W
             K::template load_x<C::SPLIT, C::SPLIT2>(tid, nb, nvol, in, R);
         __syncthreads();
         K::ypass(tid, b, nvol, sm, out, bk, scl);
+        if constexpr (C::LIN) {
+            __syncthreads();
+            Fused<C>::copy(tid, b, nvol, sm, out);
+        }
         if (nb >= nblocks) break;
         if (C::SPLIT2 < C::N0) K::template load_x<C::SPLIT2, C::N0>(tid, nb, nvol, in, R);
         __syncthreads();

@@ -20,6 +20,10 @@ void register_multi(std::vector<MultiDesc>& r)
     r.push_back(multi_desc<double, 1>("multi_c128_t640_mix", 1));
     r.push_back(multi_desc<double, 3>("multi_c128_t320_fill"));
     r.push_back(multi_desc<double, 3>("multi_c128_t320_fill_mix", 1));
+    r.push_back(multi_desc<float, 4>("multi_c64_t320_fill_lin_mix", 1));
+    r.push_back(multi_desc<float, 4>("multi_c64_t320_fill_lin"));
+    r.push_back(multi_desc<double, 5>("multi_c128_t640_lin"));
+    r.push_back(multi_desc<double, 5>("multi_c128_t640_lin_mix", 1));
     r.push_back(multi_mfma_desc<0>("multi_c64_mfma_t256_bf16x3"));
     r.push_back(multi_mfma_desc<1>("multi_c64_mfma_t256_fp16x3"));
 }

@@ -85,6 +85,28 @@ struct MultiPreset<T, 3> {
     using G3 = FusedCfg<17, 17, 17, T, -1, 1, NT, 0, 0, 1>;
     using G4 = FusedCfg<8, 8, 16, T, -1, 4, NT, 1, 0, 1>;
 };
+// Presets 3 and 1 with linear stores (FusedCfg LIN; L6: 6^3 too).  In one launch the passes' own
+// runs are shorter still, since the block order of the y pass decides them: the complex64 mix
+// below 165.6 -> 159.0 us as preset 4 (items interleaved 168.4 -> 157.3), 6^3 x 65536 alone 50.1
+// -> 46.1 and 12^3 x 8192 46.4 -> 43.9.  Complex128, as preset 5: 17^3 x 1000 43.3 -> 40.5, 12^3 x
+// 4000 52.5 -> 50.4, 8^3 x 16000 57.6 -> 55.7; 6^3 x 30000 went from 45.9 to 50.5, so it keeps
+// its own stores there.
+template <typename T, int B, int L6>
+struct LinPreset {
+    using Q = MultiPreset<T, B>;
+    static constexpr int NT = Q::NT, HN = 0;
+    template <class G, int LIN = 1>
+    using L = FusedCfg<G::N0, G::N1, G::N2, T, -1, G::VPW, NT, G::PZ, 0, 1, G::IX, LIN>;
+    using G0 = L<typename Q::G0, L6>;
+    using G1 = L<typename Q::G1>;
+    using G2 = L<typename Q::G2>;
+    using G3 = L<typename Q::G3>;
+    using G4 = L<typename Q::G4>;
+};
+template <typename T>
+struct MultiPreset<T, 4> : LinPreset<T, 3, 1> {};
+template <typename T>
+struct MultiPreset<T, 5> : LinPreset<T, 1, 0> {};
 // The staged task structure (block HBM -> LDS in one grouped read, z and y in LDS, x pass
 // LDS -> HBM with whole-line stores; the per-geometry plans of 6^3, 8^3 and 12^3 complex64
 // race to it) was built on presets 0 and 3 and measured slower in one launch: 213-228 us on
@@ -103,6 +125,7 @@ template <typename T, int PRESET>
 struct MultiCfg {
     using P = MultiPreset<T, PRESET>;
     static constexpr int NT = P::NT;
+    static constexpr bool LIN = P::G1::LIN != 0;   // some geometry stores in phase 3
     static constexpr int LDS =
         cmax(cmax(cmax(P::G0::LDS, P::G1::LDS), cmax(P::G2::LDS, P::G3::LDS)), P::G4::LDS);
     static constexpr int WPE = waves_per_eu(LDS * (int)sizeof(cx<T>), NT, 0);
@@ -113,7 +136,8 @@ struct MultiCfg {
     }
 };
 
-// Phase `ph` (0: x from HBM, 1: z, 2: y to HBM) of one block of one item.  Phases are
+// Phase `ph` (0: x from HBM, 1: z, 2: y to HBM, or to LDS for 3: copy to HBM, where the block's
+// configuration has LIN) of one block of one item.  Phases are
 // separated by workgroup barriers; no register state crosses a barrier.
 template <class C, int HN>
 FX_HD void multi_phase(int ph, int tid, long b, const MultiItem<typename C::T>& it,
@@ -132,8 +156,10 @@ FX_HD void multi_phase(int ph, int tid, long b, const MultiItem<typename C::T>& 
         K::xpass(tid, b, it.nvol, R, sm, bk);
     } else if (ph == 1) {
         K::zpass(tid, b, it.nvol, sm, bk);
-    } else {
+    } else if (ph == 2) {
         K::ypass(tid, b, it.nvol, sm, it.out, bk, it.scale, it.conj != 0);
+    } else if constexpr (C::LIN) {
+        Fused<C>::copy(tid, b, it.nvol, sm, it.out);
     }
 }
 
@@ -174,6 +200,10 @@ __device__ __forceinline__ void multi_walk(const MultiArgs<T>& a, const int2* __
         __syncthreads();
         multi_task_phase<T, PRESET>(2, tid, task, a, sm, bk);
         __syncthreads();
+        if constexpr (MultiCfg<T, PRESET>::LIN) {
+            multi_task_phase<T, PRESET>(3, tid, task, a, sm, bk);
+            __syncthreads();
+        }
         t = nt;
     }
 }

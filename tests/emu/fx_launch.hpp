@@ -111,6 +111,7 @@ hipError_t launch_fused(const void* in, void* out, long nvol, const void* bank, 
         emu_threads(C::NT, [&](int t) { K::zpass(t, b, nvol, sm, bk); });
         emu_threads(C::NT, [&](int t) { K::ypass(t, b, nvol, sm, bk); });
         emu_threads(C::NT, [&](int t) { K::xpass(t, b, nvol, sm, (cx<T>*)out, bk, (T)scl); });
+        if constexpr (C::LIN) emu_threads(C::NT, [&](int t) { K::copy(t, b, nvol, sm, (cx<T>*)out); });
         if (!lds.guards_ok() && g_emu_bad_block < 0) g_emu_bad_block = b;
     }
     return hipSuccess;
@@ -156,6 +157,8 @@ hipError_t launch_fpipe(const void* in, void* out, long nvol, const void* bank, 
                     K::template load_x<SPLIT, SPLIT2>(t, nb, nvol, src, R[w][t].r);
                 });
             emu_threads(C::NT, [&](int t) { K::ypass(t, b, nvol, sm, dst, bk, (T)scl); });
+            if constexpr (C::LIN)
+                emu_threads(C::NT, [&](int t) { Fused<C>::copy(t, b, nvol, sm, dst); });
             if (SPLIT2 < C::N0 && nb < nblocks)
                 emu_threads(C::NT, [&](int t) {
                     K::template load_x<SPLIT2, C::N0>(t, nb, nvol, src, R[w][t].r);

@@ -1,6 +1,6 @@
 // TEST INFRASTRUCTURE: host emulation of the mixed-batch launcher (see fx_launch.hpp for the
 // emulation rules).  The grid is 3 workgroups walking the task list round-robin; each task
-// runs its three phases over all threads in barrier order, LDS re-poisoned per task.
+// runs its three phases (four with linear stores) over all threads in barrier order, LDS re-poisoned per task.
 #pragma once
 
 namespace fx {
@@ -20,7 +20,7 @@ hipError_t launch_multi(const void* args, const int2* tasks, int ntasks, const v
         [&](long, long t, long) {
             lds.poison();
             cx<T>* sm = lds.data();
-            for (int ph = 0; ph < 3; ++ph)
+            for (int ph = 0; ph < (M::LIN ? 4 : 3); ++ph)
                 emu_threads(M::NT, [&](int tid) { multi_task_phase<T, PRESET>(ph, tid, tasks[t], a, sm, bk); });
             if (!lds.guards_ok() && g_emu_bad_block < 0) g_emu_bad_block = t;
         });
