@@ -245,10 +245,13 @@ static const KernelDesc* race(const std::vector<const KernelDesc*>& cands, int n
             for (const KernelDesc* k : cands) ts.push_back(Trial{k, 0, 0, 1e30});
             run_trials(rig, ts);
             // A later candidate must beat the incumbent by more than 1.5% (above the
-            // run-to-run spread of one trial), so near-ties resolve the same way each time, to
-            // the earlier-registered variant.
+            // run-to-run spread of one trial) and a tenth of a microsecond more, so near-ties
+            // resolve the same way each time, to the earlier-registered variant.  The tenth
+            // is for kernels that last as long as a launch: there a full queue hides a
+            // kernel's start, which a paced caller pays (6^3 complex128 x 289: 3.74 us here to
+            // the staged kernel's 3.82, and 4.5 to 3.9 launched from Python).
             for (const Trial& t : ts)
-                if (t.best < 1e29 && (wt > 1e29 || t.best < 0.985 * wt)) {
+                if (t.best < 1e29 && (wt > 1e29 || t.best < 0.985 * wt - 0.1e-6)) {
                     wt = t.best;
                     win = t.k;
                 }
