@@ -3,11 +3,18 @@
 
 namespace fx {
 
-template <typename T, int PRESET>
-long multi_launch_grid(long ntasks)
+template <typename T, int PRESET, bool G17 = true>
+long multi_grid(long ntasks)
 {
-    static const int per = resident_per_cu(k_multi<T, PRESET>, MultiCfg<T, PRESET>::NT);
+    static const int per = resident_per_cu(k_multi<T, PRESET, G17>, MultiCfg<T, PRESET>::NT);
     return persistent_grid(per, 8, ntasks);
+}
+template <typename T, int PRESET>
+long multi_launch_grid(long ntasks, bool g17)
+{
+    if constexpr (kMultiSmall<PRESET>)
+        if (!g17) return multi_grid<T, PRESET, false>(ntasks);
+    return multi_grid<T, PRESET>(ntasks);
 }
 
 template <typename T, int PRESET>
@@ -16,10 +23,14 @@ hipError_t launch_multi(const void* args, const int2* tasks, int ntasks, const v
 {
     using M = MultiCfg<T, PRESET>;
     if (ntasks <= 0) return hipSuccess;
-    const long grid = multi_launch_grid<T, PRESET>(ntasks);
-    hipLaunchKernelGGL((k_multi<T, PRESET>), dim3((unsigned)grid), dim3(M::NT), 0, stream,
-                       *(const MultiArgs<T>*)args, tasks, ntasks, (const Bank<T>*)bank,
-                       claim_counter(work, grid, ntasks));
+    const MultiArgs<T>& a = *(const MultiArgs<T>*)args;
+    const bool g17 = !kMultiSmall<PRESET> || multi_has17(a);
+    const long grid = multi_launch_grid<T, PRESET>(ntasks, g17);
+    auto* k = k_multi<T, PRESET>;
+    if constexpr (kMultiSmall<PRESET>)
+        if (!g17) k = k_multi<T, PRESET, false>;
+    hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(M::NT), 0, stream, a, tasks, ntasks,
+                       (const Bank<T>*)bank, claim_counter(work, grid, ntasks));
     return hipGetLastError();
 }
 

@@ -15,7 +15,7 @@ hipError_t launch_multi_mfma(const void* args, const int2* tasks, int ntasks, co
 }
 
 // One workgroup per task.
-inline long multi_mfma_grid(long ntasks) { return ntasks; }
+inline long multi_mfma_grid(long ntasks, bool) { return ntasks; }
 
 template <int SPLIT>
 MultiDesc multi_mfma_desc(const char* name)

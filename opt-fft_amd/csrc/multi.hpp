@@ -107,6 +107,48 @@ template <typename T>
 struct MultiPreset<T, 4> : LinPreset<T, 3, 1> {};
 template <typename T>
 struct MultiPreset<T, 5> : LinPreset<T, 1, 0> {};
+// Small blocks, sized without regard to 17^3: 192 threads and one 12^3 volume (30 KB at
+// complex128), or 320 / 384 and two of complex64.  These presets have a second kernel for
+// launches without 17^3 items, whose LDS and registers are those of the other geometries: at
+// complex128 five workgroups a CU (88 VGPRs) where 17^3 allows two (184), at complex64 five of
+// 320-384 threads instead of four.  Against the best earlier preset (us):
+//   complex128, 7:  12^3 x 2401 with 6^3 x 40  33.5 -> 27.4; 6^3 x 2842, 8^3 x 8442  36.3 -> 31.0;
+//                   6^3 x 20000, 8^3 x 8000, 12^3 x 3000  86.1 -> 78.8; a hundredth of it 9.1 -> 8.3
+//   complex64, 8/9: the same 17.9 -> 12.4 / 13.6; 19.9 -> 17.0 / 16.8; 43.7 -> 40.0 / 40.3; 6.4 -> 6.1
+// With 17^3 in the mix (289 lines on 192 threads) preset 6 is ahead at complex128 where the
+// small geometries hold most of the bytes, 6^3 x 10000, 8^3 x 4000, 12^3 x 1500, 17^3 x 500
+// 65.7 -> 61.2, and 9 at complex64, 12^3 x 4854 with 17^3 x 258 36.3 -> 35.7; 8x8x16 x 6000 with
+// 17^3 x 100 takes 58.2 (54.4 as preset 3).  Not registered: 6 and 7 with the items interleaved
+// (127-140 us in place of 61-68 at the mix above), 9 at complex128 (two workgroups a CU: 42.0
+// to 31.0 at 6^3 with 8^3), 192 threads at complex64 (within 2% of 8).
+template <typename T>
+struct MultiPreset<T, 6> {
+    static constexpr int NT = 192;
+    static constexpr int HN = 0;
+    using G0 = FusedCfg<6, 6, 6, T, -1, 5, NT, 1, 0, 1>;
+    using G1 = FusedCfg<8, 8, 8, T, -1, 3, NT, 1, 0, 1>;
+    using G2 = FusedCfg<12, 12, 12, T, -1, 1, NT, 1, 0, 1>;
+    using G3 = FusedCfg<17, 17, 17, T, -1, 1, NT, 0, 0, 1>;
+    using G4 = FusedCfg<8, 8, 16, T, -1, 1, NT, 1, 0, 1>;
+};
+template <typename T>
+struct MultiPreset<T, 7> : LinPreset<T, 6, 1> {};
+template <typename T>
+struct MultiPreset<T, 8> : LinPreset<T, 0, 1> {};
+template <typename T>
+struct MultiPreset<T, 10> {   // the blocks of preset 9
+    static constexpr int NT = 384;
+    static constexpr int HN = 0;
+    using G0 = FusedCfg<6, 6, 6, T, -1, 10, NT, 1, 0, 1>;
+    using G1 = FusedCfg<8, 8, 8, T, -1, 6, NT, 1, 0, 1>;
+    using G2 = FusedCfg<12, 12, 12, T, -1, 2, NT, 1, 0, 1>;
+    using G3 = FusedCfg<17, 17, 17, T, -1, 1, NT, 0, 0, 1>;
+    using G4 = FusedCfg<8, 8, 16, T, -1, 3, NT, 1, 0, 1>;
+};
+template <typename T>
+struct MultiPreset<T, 9> : LinPreset<T, 10, 1> {};
+template <int PRESET>
+constexpr bool kMultiSmall = PRESET >= 6;   // has the second kernel
 // The staged task structure (block HBM -> LDS in one grouped read, z and y in LDS, x pass
 // LDS -> HBM with whole-line stores; the per-geometry plans of 6^3, 8^3 and 12^3 complex64
 // race to it) was built on presets 0 and 3 and measured slower in one launch: 213-228 us on
@@ -121,13 +163,15 @@ struct MultiPreset<T, 5> : LinPreset<T, 1, 0> {};
 
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 
-template <typename T, int PRESET>
+// G17: 17^3 items may occur.  Without them the workgroup's LDS and registers are those of the
+// other geometries.
+template <typename T, int PRESET, bool G17 = true>
 struct MultiCfg {
     using P = MultiPreset<T, PRESET>;
     static constexpr int NT = P::NT;
     static constexpr bool LIN = P::G1::LIN != 0;   // some geometry stores in phase 3
     static constexpr int LDS =
-        cmax(cmax(cmax(P::G0::LDS, P::G1::LDS), cmax(P::G2::LDS, P::G3::LDS)), P::G4::LDS);
+        cmax(cmax(cmax(P::G0::LDS, P::G1::LDS), cmax(P::G2::LDS, G17 ? P::G3::LDS : 0)), P::G4::LDS);
     static constexpr int WPE = waves_per_eu(LDS * (int)sizeof(cx<T>), NT, 0);
     static constexpr int vpw(int code)
     {
@@ -163,7 +207,7 @@ FX_HD void multi_phase(int ph, int tid, long b, const MultiItem<typename C::T>& 
     }
 }
 
-template <typename T, int PRESET>
+template <typename T, int PRESET, bool G17 = true>
 FX_HD void multi_task_phase(int ph, int tid, int2 task, const MultiArgs<T>& a, cx<T>* sm,
                             const Bank<T>* __restrict__ bk)
 {
@@ -173,7 +217,9 @@ FX_HD void multi_task_phase(int ph, int tid, int2 task, const MultiArgs<T>& a, c
     case 0: multi_phase<typename P::G0, P::HN>(ph, tid, task.y, it, sm, bk); break;
     case 1: multi_phase<typename P::G1, P::HN>(ph, tid, task.y, it, sm, bk); break;
     case 2: multi_phase<typename P::G2, P::HN>(ph, tid, task.y, it, sm, bk); break;
-    case 3: multi_phase<typename P::G3, P::HN>(ph, tid, task.y, it, sm, bk); break;
+    case 3:
+        if constexpr (G17) multi_phase<typename P::G3, P::HN>(ph, tid, task.y, it, sm, bk);
+        break;
     default: multi_phase<typename P::G4, P::HN>(ph, tid, task.y, it, sm, bk); break;
     }
 }
@@ -181,7 +227,7 @@ FX_HD void multi_task_phase(int ph, int tid, int2 task, const MultiArgs<T>& a, c
 // Walk the task list: the first task is blockIdx.x, the next ones are claimed from `work`
 // (NULL: a fixed stride of gridDim.x).  The claim is issued before phase 0 and published to
 // the workgroup at the first barrier.
-template <typename T, int PRESET>
+template <typename T, int PRESET, bool G17 = true>
 __device__ __forceinline__ void multi_walk(const MultiArgs<T>& a, const int2* __restrict__ tasks,
                                            int ntasks, const Bank<T>* __restrict__ bk,
                                            unsigned* work, cx<T>* sm, long* s_next)
@@ -192,32 +238,32 @@ __device__ __forceinline__ void multi_walk(const MultiArgs<T>& a, const int2* __
         long claim = 0;
         if (tid == 0) claim = claim_block(work, ntasks, t);
         const int2 task = tasks[t];
-        multi_task_phase<T, PRESET>(0, tid, task, a, sm, bk);
+        multi_task_phase<T, PRESET, G17>(0, tid, task, a, sm, bk);
         if (tid == 0) *s_next = claim;
         __syncthreads();
         const long nt = *s_next;
-        multi_task_phase<T, PRESET>(1, tid, task, a, sm, bk);
+        multi_task_phase<T, PRESET, G17>(1, tid, task, a, sm, bk);
         __syncthreads();
-        multi_task_phase<T, PRESET>(2, tid, task, a, sm, bk);
+        multi_task_phase<T, PRESET, G17>(2, tid, task, a, sm, bk);
         __syncthreads();
         if constexpr (MultiCfg<T, PRESET>::LIN) {
-            multi_task_phase<T, PRESET>(3, tid, task, a, sm, bk);
+            multi_task_phase<T, PRESET, G17>(3, tid, task, a, sm, bk);
             __syncthreads();
         }
         t = nt;
     }
 }
 
-template <typename T, int PRESET>
-__global__ void __launch_bounds__((MultiCfg<T, PRESET>::NT))
-    __attribute__((amdgpu_waves_per_eu(MultiCfg<T, PRESET>::WPE, 8)))
+template <typename T, int PRESET, bool G17 = true>
+__global__ void __launch_bounds__((MultiCfg<T, PRESET, G17>::NT))
+    __attribute__((amdgpu_waves_per_eu(MultiCfg<T, PRESET, G17>::WPE, 8)))
     k_multi(const MultiArgs<T> a, const int2* __restrict__ tasks, int ntasks,
             const Bank<T>* __restrict__ bk, unsigned* __restrict__ work)
 {
-    using M = MultiCfg<T, PRESET>;
+    using M = MultiCfg<T, PRESET, G17>;
     __shared__ cx<T> sm[M::LDS];
     __shared__ long s_next;
-    multi_walk<T, PRESET>(a, tasks, ntasks, bk, work, sm, &s_next);
+    multi_walk<T, PRESET, G17>(a, tasks, ntasks, bk, work, sm, &s_next);
 }
 
 // Same kernel with the items, the task count and the task list read from device memory, so a
@@ -245,6 +291,15 @@ __global__ void __launch_bounds__((MultiCfg<T, PRESET>::NT))
                           sm, &s_next);
 }
 
+// Does any item of a launch hold 17^3 volumes?
+template <typename T>
+bool multi_has17(const MultiArgs<T>& a)
+{
+    for (const MultiItem<T>& it : a.item)
+        if (it.code == 3 && it.nvol > 0) return true;
+    return false;
+}
+
 // Registry entry of a multi kernel.
 // `work`: claim counter as for LaunchFn (registry.hpp).
 typedef hipError_t (*MultiLaunchFn)(const void* args, const int2* tasks, int ntasks,
@@ -263,7 +318,8 @@ struct MultiDesc {
     MultiDevLaunchFn launch_dev;  // NULL: no descriptor form
     int (*resident_grid)();  // persistent grid of the descriptor form on the current device
     int algo = 0;            // as KernelDesc::algo: 0 FFT, 1 / 2 matrix-core bf16 / fp16
-    long (*launch_grid)(long ntasks) = nullptr;  // workgroups `launch` starts for ntasks
+    // Workgroups `launch` starts for ntasks, of items with or without 17^3.
+    long (*launch_grid)(long ntasks, bool g17) = nullptr;
     int order = 0;  // task order (multi_tasks): 0 heaviest first, 1 items interleaved
 };
 

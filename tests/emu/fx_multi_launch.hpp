@@ -5,11 +5,11 @@
 
 namespace fx {
 
-template <typename T, int PRESET>
-hipError_t launch_multi(const void* args, const int2* tasks, int ntasks, const void* bank,
-                        unsigned* work, hipStream_t)
+template <typename T, int PRESET, bool G17>
+hipError_t launch_multi_as(const void* args, const int2* tasks, int ntasks, const void* bank,
+                           unsigned* work)
 {
-    using M = MultiCfg<T, PRESET>;
+    using M = MultiCfg<T, PRESET, G17>;
     const MultiArgs<T>& a = *(const MultiArgs<T>*)args;
     const Bank<T>* bk = (const Bank<T>*)bank;
     if (ntasks <= 0) return hipSuccess;
@@ -21,10 +21,19 @@ hipError_t launch_multi(const void* args, const int2* tasks, int ntasks, const v
             lds.poison();
             cx<T>* sm = lds.data();
             for (int ph = 0; ph < (M::LIN ? 4 : 3); ++ph)
-                emu_threads(M::NT, [&](int tid) { multi_task_phase<T, PRESET>(ph, tid, tasks[t], a, sm, bk); });
+                emu_threads(M::NT, [&](int tid) { multi_task_phase<T, PRESET, G17>(ph, tid, tasks[t], a, sm, bk); });
             if (!lds.guards_ok() && g_emu_bad_block < 0) g_emu_bad_block = t;
         });
     return hipSuccess;
+}
+
+template <typename T, int PRESET>
+hipError_t launch_multi(const void* args, const int2* tasks, int ntasks, const void* bank,
+                        unsigned* work, hipStream_t)
+{
+    if (kMultiSmall<PRESET> && !multi_has17(*(const MultiArgs<T>*)args))
+        return launch_multi_as<T, PRESET, false>(args, tasks, ntasks, bank, work);
+    return launch_multi_as<T, PRESET, true>(args, tasks, ntasks, bank, work);
 }
 
 template <typename T, int PRESET>
