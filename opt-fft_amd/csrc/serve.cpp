@@ -484,13 +484,20 @@ extern "C" fft3d_srv* fft3d_srv_create(const fft3d_srv_config* cfg)
         ok = hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
         if (ok) s->event_pool.push_back(e);
     }
+    // The mixed kernel of each precision.  complex64, whole-line stores: 6^3 x 2000 with 17^3 x 300
+    // takes 11.9 us (320 threads storing a line's points 14.3), 6^3 x 2000 with 12^3 x 900 and
+    // 17^3 x 800 24.5 (25.5); p99 of the serving mix at 195,000 requests/s 3.1 -> 1.7 ms (medians
+    // of five runs).  complex128: 17^3 x 6, 6^3 x 1838 and 12^3 x 28 take 9.6 us as below, 11.9
+    // with 192 threads, 12.8 with 640; under load 640 with whole-line stores measured better in
+    // one combination and worse in another.
+    static const char* const mixed[2] = {"multi_c128_t320", "multi_c64_t384_lin"};
     for (int prec = 0; prec < 2 && ok; ++prec) {
         std::vector<unsigned char> img;
         bank_host_image(prec, img);
         ok = hipMalloc(&s->bank[prec], img.size()) == hipSuccess &&
              hipMemcpy(s->bank[prec], img.data(), img.size(), hipMemcpyHostToDevice) == hipSuccess;
         for (const MultiDesc& d : multi_registry())
-            if (d.prec == prec && d.algo == 0 && d.launch_dev && !s->mk[prec]) s->mk[prec] = &d;
+            if (d.prec == prec && d.launch_dev && !strcmp(d.name, mixed[prec])) s->mk[prec] = &d;
         ok = ok && s->mk[prec] && make_slots(s, prec, cfg->streams);
     }
     // Plans for every geometry, both precisions and directions (the plain modes use them
