@@ -104,9 +104,10 @@ typedef struct fft3d_mx_plan_info {
     int n0, n1, n2, batch, direction, precision;
     int kind;            /* 0 fused (volume resident in LDS), 1 pencil (two passes) */
     int volumes_per_wg;  /* fused: volumes per workgroup; pencil: slabs per workgroup */
-    int threads;         /* workgroup size of the main kernel */
+    int threads;         /* workgroup size of the main kernel (of several forms, "..._v1rounds":
+                            the one that runs full rounds) */
     int variant;         /* line-algorithm variant (L=17: 0 Rader, 1 folded dense) */
-    size_t lds_bytes;    /* LDS per workgroup of the main kernel */
+    size_t lds_bytes;    /* LDS per workgroup of the main kernel (as for threads) */
     double tune_us;      /* create-time race result of the winner (0 if no race) */
     char kernel[96];     /* kernel name */
     long small_max;      /* executes of at most this many volumes use kernel_small (0: none) */
@@ -115,6 +116,9 @@ typedef struct fft3d_mx_plan_info {
        executes that many and fewer through plane_17x17x17_*, whatever the classes above.) */
 } fft3d_mx_plan_info;
 int fft3d_mx_plan_get_info(const fft3d_mx_plan *plan, fft3d_mx_plan_info *info);
+/* Name of the kernel that an execute of `batch` volumes launches, whichever class it falls in;
+ * NULL for a NULL plan or a batch outside [1, the planned batch]. */
+const char *fft3d_mx_plan_kernel_at(const fft3d_mx_plan *plan, long batch);
 
 /* Kernel registry enumeration: every compiled kernel variant. */
 int fft3d_mx_kernel_count(void);

@@ -602,6 +602,15 @@ extern "C" int fft3d_mx_plan_get_info(const fft3d_mx_plan* p, fft3d_mx_plan_info
     return FFT3D_MX_OK;
 }
 
+extern "C" const char* fft3d_mx_plan_kernel_at(const fft3d_mx_plan* p, long batch)
+{
+    if (!p || batch < 1 || batch > p->batch) {
+        fail(FFT3D_MX_EINVAL, "fft3d_mx_plan_kernel_at: NULL plan or batch %ld outside it", batch);
+        return nullptr;
+    }
+    return kernel_for(p, batch)->name;
+}
+
 extern "C" int fft3d_mx_kernel_count(void) { return (int)registry().size(); }
 
 extern "C" const char* fft3d_mx_kernel_name(int i, int* n0, int* n1, int* n2, int* precision,

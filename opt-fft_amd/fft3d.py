@@ -37,8 +37,8 @@ EXPORTED = [
     "fft3d_mx_last_error", "fft3d_mx_clear_error", "fft3d_mx_supports", "fft3d_mx_create",
     "fft3d_mx_create_named", "fft3d_mx_execute", "fft3d_mx_execute_n",
     "fft3d_mx_execute_chain", "fft3d_mx_destroy",
-    "fft3d_mx_plan_get_info", "fft3d_mx_kernel_count", "fft3d_mx_kernel_name",
-    "fft3d_mx_bank_image", "fft3d_mx_volume_bytes", "fft3d_mx_execute_noalloc",
+    "fft3d_mx_plan_get_info", "fft3d_mx_plan_kernel_at", "fft3d_mx_kernel_count",
+    "fft3d_mx_kernel_name", "fft3d_mx_bank_image", "fft3d_mx_volume_bytes", "fft3d_mx_execute_noalloc",
     "fft3d_mx_multi_create", "fft3d_mx_multi_execute", "fft3d_mx_multi_get_info",
     "fft3d_mx_multi_destroy",
     "fft3d_srv_create", "fft3d_srv_submit", "fft3d_srv_wait", "fft3d_srv_run_trace",
@@ -120,6 +120,8 @@ def load():
         L.fft3d_mx_execute_chain.argtypes = [vp, vp, vp, vp, ci, ctypes.c_double, vp]
         L.fft3d_mx_destroy.argtypes = [vp]
         L.fft3d_mx_plan_get_info.argtypes = [vp, ctypes.POINTER(PlanInfo)]
+        L.fft3d_mx_plan_kernel_at.argtypes = [vp, cl]
+        L.fft3d_mx_plan_kernel_at.restype = ctypes.c_char_p
         L.fft3d_mx_kernel_name.argtypes = [ci, ip, ip, ip, ip, ip]
         L.fft3d_mx_kernel_name.restype = ctypes.c_char_p
         L.fft3d_mx_bank_image.argtypes = [ci, vp, cs, ctypes.POINTER(cs)]
@@ -224,6 +226,13 @@ class Plan:
         """(kernel, max volumes) of the small-batch class, or None."""
         inf = self.info()
         return (inf.kernel_small.decode(), inf.small_max) if inf.small_max else None
+
+    def kernel_at(self, batch):
+        """The kernel that an execute of `batch` volumes launches."""
+        name = load().fft3d_mx_plan_kernel_at(self.handle, int(batch))
+        if name is None:
+            raise ValueError(last_error())
+        return name.decode()
 
     def execute(self, din, dout, batch=None, stream=None):
         """Enqueue on `stream` (hip.Stream, raw handle or None) with device addresses."""
