@@ -68,7 +68,8 @@ int fft3d_mx_supports(int n0, int n1, int n2, int precision);
  * cached per process, and in the file named by $FFT3D_MX_WISDOM when that is set).  For
  * batch >= 16 the race also runs at batch / 8, and executes of at most
  * sqrt(batch * (batch / 8)) volumes use that winner if it differs (plan_info's
- * kernel_small, small_max).  $FFT3D_MX_KERNEL=<name> forces a kernel by name.  NULL on
+ * kernel_small, small_max).  17^3 batches below the limit given at plan_info are not raced.
+ * $FFT3D_MX_KERNEL=<name> forces a kernel by name.  NULL on
  * failure. */
 fft3d_mx_plan *fft3d_mx_create(int n0, int n1, int n2, int batch, int direction,
                                int precision, unsigned flags);
@@ -112,8 +113,9 @@ typedef struct fft3d_mx_plan_info {
     char kernel[96];     /* kernel name */
     long small_max;      /* executes of at most this many volumes use kernel_small (0: none) */
     char kernel_small[96];  /* small-batch kernel name ("" if none) */
-    /* (17^3: a raced plan of more than 32 (complex128) or 48 (complex64) volumes, on 256 CUs,
-       executes that many and fewer through plane_17x17x17_*, whatever the classes above.) */
+    /* (17^3: up to 32 volumes (complex128; complex64 48), on 256 CUs, execute through
+       plane_17x17x17_*, whatever the classes above, unless the plan's kernel is forced or
+       FFT3D_MX_NO_TUNE is set; fft3d_mx_plan_kernel_at tells.) */
 } fft3d_mx_plan_info;
 int fft3d_mx_plan_get_info(const fft3d_mx_plan *plan, fft3d_mx_plan_info *info);
 /* Name of the kernel that an execute of `batch` volumes launches, whichever class it falls in;

@@ -280,7 +280,7 @@ struct fft3d_mx_plan {
     const KernelDesc* k_small;
     long small_max;
     // Tiny class (KernelDesc::tiny): executes of at most tiny_max volumes launch k_tiny when it
-    // is not NULL (plans whose kernel was raced, at batches above tiny_max).
+    // is not NULL (raced plans of batches above tiny_max; k itself is the tiny kernel below).
     const KernelDesc* k_tiny;
     long tiny_max;
     void* bank;
@@ -451,8 +451,25 @@ static fft3d_mx_plan* create_impl(int n0, int n1, int n2, int batch, int directi
     p->k_tiny = nullptr;
     p->tiny_max = 0;
     if (!pick) {
-        if (cands.size() == 1 || (flags & FFT3D_MX_NO_TUNE) || batch == 0) {
-            pick = cands[0];
+        // A kernel with a tiny class serves the batches of that class and takes part in no race:
+        // the small-batch class spans batches up to 2.8 times the raced one, and a recorded
+        // verdict a power of two, so its win at 32 volumes would carry it to 63 or 90 (17^3
+        // complex128 x 64: 11.4 us to the volume kernel's 8.4).
+        std::vector<const KernelDesc*> raced;
+        const KernelDesc* tiny = nullptr;
+        long tiny_max = 0;
+        for (const KernelDesc* k : cands) {
+            if (k->tiny > 0) {
+                tiny = k;
+                tiny_max = (long)k->tiny * p->cus / 256;
+            } else {
+                raced.push_back(k);
+            }
+        }
+        if (raced.size() == 1 || (flags & FFT3D_MX_NO_TUNE) || batch == 0) {
+            pick = raced[0];
+        } else if (batch <= tiny_max) {
+            pick = tiny;
         } else {
             // The race (or the wisdom it left) at the planned batch, and at an eighth of it:
             // a kernel that fills the device at 512 volumes (one workgroup per volume) can
@@ -463,30 +480,27 @@ static fft3d_mx_plan* create_impl(int n0, int n1, int n2, int batch, int directi
                 const std::string key = wisdom_key(n0, n1, n2, precision, direction, b, algo);
                 auto it = g_wisdom.find(key);
                 if (it != g_wisdom.end())
-                    for (const KernelDesc* k : cands)
+                    for (const KernelDesc* k : raced)
                         if (it->second == k->name) return k;
                 double best_s = 0.0;
-                const KernelDesc* k = race(cands, n0, n1, n2, precision, b, p->bank, p->work,
+                const KernelDesc* k = race(raced, n0, n1, n2, precision, b, p->bank, p->work,
                                            &best_s);
                 if (tune_us) *tune_us = best_s * 1e6;
                 if (best_s > 0) wisdom_store_locked(key, k->name);
                 return k;
             };
             pick = pick_at(batch, &p->tune_us);
-            if (batch >= 16) {
-                const long bs = batch / 8;
+            const long bs = batch / 8, small_max = (long)std::sqrt((double)batch * (double)bs);
+            if (batch >= 16 && small_max > tiny_max) {
                 const KernelDesc* ks = pick_at(bs, nullptr);
                 if (ks != pick) {
                     p->k_small = ks;
-                    p->small_max = (long)std::sqrt((double)batch * (double)bs);
+                    p->small_max = small_max;
                 }
             }
-            for (const KernelDesc* k : cands) {
-                const long most = (long)k->tiny * p->cus / 256;
-                if (most > 0 && batch > most) {
-                    p->k_tiny = k;
-                    p->tiny_max = most;
-                }
+            if (tiny_max > 0) {
+                p->k_tiny = tiny;
+                p->tiny_max = tiny_max;
             }
         }
     }

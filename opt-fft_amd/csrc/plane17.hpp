@@ -10,9 +10,15 @@
 //       plane 0 -> plane 1 -> HBM, runs of 17 elements.
 // A workgroup an output plane reads the volume 17 times (from L2) and spends about four times the
 // arithmetic of whole lines, so the volume kernel takes over when its workgroups begin to fill
-// the device (us, complex128: this kernel / the quickest volume kernel; 3.3 is the host's issue):
-//   x 1 3.6 / 6.6   x 8 3.9 / 6.9   x 16 5.3 / 8.8   x 32 7.8 / 9.3   x 48 11.1 / 10.1
-//   complex64: x 1 3.5 / 5.8   x 16 4.3 / 6.3   x 32 5.4 / 6.7   x 48 6.2 / 6.8   x 64 7.2 / 6.9
+// the device (us a launch back to back, this kernel / the quickest volume kernel, over 64 MB of
+// buffers in turn; 3.3 is the host's issue).  Times step where another round of workgroups
+// begins, past 8, 24 and 32 volumes in complex128:
+//   x 1 3.9 / 6.8   x 8 4.1 / 7.1   x 24 5.5 / 8.0   x 32 7.4 / 8.2   x 36 8.1 / 8.2   x 48 9.6 / 8.3
+//   over 1 GB: x 1 4.5 / 7.2   x 24 6.8 / 8.5   x 32 8.4 / 8.7   x 36 9.4 / 8.8   x 48 11.3 / 8.9
+//   complex64: x 1 3.8 / 5.7   x 24 4.5 / 6.4   x 40 5.4 / 6.5   x 48 6.2 / 6.5   x 64 7.0 / 6.6
+//   over 1 GB: x 1 3.8 / 5.8   x 24 5.1 / 6.7   x 40 6.3 / 6.9   x 48 7.1 / 7.0   x 64 8.2 / 7.2
+// and waited for one by one: complex128 x 24 16.5 / 18.0, x 32 18.3 / 18.1; complex64 x 40 16.3 /
+// 16.8, x 48 17.5 / 17.2;
 // hence TINY, 32 and 48 volumes on 256 CUs.
 #pragma once
 #include "codelets.hpp"

@@ -36,8 +36,9 @@ struct KernelDesc {
     const char* name;
     LaunchFn launch;
     int algo = 0;    // 0 exact FP FFT; 1 DFT matrix on MFMA, split bf16; 2 split fp16
-    // Volumes per 256 CUs up to which this kernel is the quickest of its geometry: plans whose
-    // kernel was raced launch it there, whatever won at their batch.  0: no such class.
+    // Volumes per 256 CUs up to which this kernel is the quickest of its geometry: plans without a
+    // forced kernel and FFT3D_MX_NO_TUNE launch it there and only there; it is not raced.  0: no
+    // such class.
     int tiny = 0;
 };
 
