@@ -13,7 +13,7 @@
 #include "multi.hpp"
 #include "multi_tasks.hpp"
 #include "plan_internal.hpp"
-
+#include "race_hip.hpp"
 
 using namespace fx;
 
@@ -86,11 +86,14 @@ static const MultiDesc* multi_race(fft3d_mx_multi* m, const std::vector<const Mu
         total += (size_t)kMultiShape[g][0] * kMultiShape[g][1] * kMultiShape[g][2] * elem * m->batch[i];
     }
     const double shrink = total > (256ull << 20) ? (double)(256ull << 20) / (double)total : 1.0;
-    // Sets of buffers in turn, 512 MiB of them together, 16 at most: stores of part of a line cost
-    // little while the line is in a cache and much otherwise (6^3 x 200, 8^3 x 800, 12^3 x 300 as
-    // multi_c128_t192: 8.4 us over 256 MB, 10.3 over 384).
+    // Sets of buffers in turn, 256 MiB of input in all and at least two, 16 at most, and as much
+    // output: stores of part of a line cost little while the line is in a cache and much otherwise
+    // (6^3 x 200, 8^3 x 800, 12^3 x 300 as multi_c128_t192: 8.4 us over 256 MB, 10.3 over 384), and
+    // one set of 256 MiB leaves parts of itself there (the complex64 mix 6^3 x 65536, 8^3 x 32768,
+    // 12^3 x 8192, 17^3 x 2048: multi_c64_t320_fill_lin 85 us to .._lin_mix's 108 over one set, 102
+    // to 100 over two; executed it takes 164 to 161).
     const size_t one = std::max<size_t>(1, std::min<size_t>(total, 256ull << 20));
-    int sets = (int)std::max<size_t>(1, std::min<size_t>(16, (256ull << 20) / one));
+    int sets = (int)std::max<size_t>(2, std::min<size_t>(16, (256ull << 20) / one));
     std::vector<void*> bufs;
     std::vector<std::vector<const void*>> ins(sets, std::vector<const void*>(m->nitems));
     std::vector<std::vector<void*>> outs(sets, std::vector<void*>(m->nitems));
@@ -127,52 +130,41 @@ static const MultiDesc* multi_race(fft3d_mx_multi* m, const std::vector<const Mu
         int saved[kMultiMaxItems];
         std::memcpy(saved, m->batch, sizeof saved);
         std::memcpy(m->batch, rb, sizeof(int) * m->nitems);
-        hipEvent_t e0, e1;
+        std::vector<int2*> tasks(cands.size(), nullptr);
+        std::vector<int> ntasks(cands.size(), -1);
+        for (size_t i = 0; i < cands.size(); ++i) {
+            std::vector<int2> t;
+            multi_tasks(*cands[i], m->code, m->batch, m->nitems, elem, t);
+            if (upload_tasks(t, &tasks[i]) == FFT3D_MX_OK) ntasks[i] = (int)t.size();
+        }
         hipStream_t s;
-        double best = 1e30;
-        const bool have_s = hipStreamCreate(&s) == hipSuccess;
-        const bool have_e0 = have_s && hipEventCreate(&e0) == hipSuccess;
-        const bool have_e1 = have_e0 && hipEventCreate(&e1) == hipSuccess;
-        if (have_e1) {
-            for (const MultiDesc* k : cands) {
-                std::vector<int2> t;
-                multi_tasks(*k, m->code, m->batch, m->nitems, elem, t);
-                int2* dt = nullptr;
-                if (upload_tasks(t, &dt) != FFT3D_MX_OK) continue;
+        if (hipStreamCreate(&s) == hipSuccess) {
+            {
+                RaceEvents ev(cands.size());
                 int w = 0;
-                auto launch = [&] {
-                    const int c = w++ % sets;
-                    return multi_launch(m, k, dt, (int)t.size(), ins[c].data(), outs[c].data(),
-                                        m->work, s) == hipSuccess;
+                auto launch = [&](size_t k, int n) {
+                    for (int i = 0; i < n; ++i) {
+                        const int c = w++ % sets;
+                        if (ntasks[k] < 0 || multi_launch(m, cands[k], tasks[k], ntasks[k], ins[c].data(),
+                                                          outs[c].data(), m->work, s) != hipSuccess)
+                            return false;
+                    }
+                    return true;
                 };
-                bool good = launch() && launch();
-                // A group of three launches sizes the others to 150 us: three launches of a small
-                // mix last 20, and event jitter then chose among presets 10% apart.
-                double kt = 1e30;
-                int n = 3;
-                for (int g = 0; g < (n == 3 ? 4 : 3) && good; ++g) {
-                    good = hipEventRecord(e0, s) == hipSuccess;
-                    for (int r = 0; r < n && good; ++r) good = launch();
-                    good = good && hipEventRecord(e1, s) == hipSuccess && hipEventSynchronize(e1) == hipSuccess;
-                    float ms = 0.f;
-                    good = good && hipEventElapsedTime(&ms, e0, e1) == hipSuccess;
-                    const double per = (double)ms / n;
-                    if (g == 0) n = std::max(3, std::min(64, (int)(0.15 / std::max(per, 1e-3))));
-                    if (good && (g > 0 || n == 3)) kt = std::min(kt, per);
-                    if (per > 1.3 * best) break;   // out
+                std::vector<Trial> ts(cands.size());
+                if (ev.ok) {
+                    run_trials(ts, kMultiRace, sets * one >= (128ull << 20) ? sets : 1, launch,
+                               [&](const std::vector<Trial>& c, std::vector<double>& t) {
+                                   return ev.round(c, t, s, launch);
+                               });
+                    const int best = race_winner(ts);
+                    if (best >= 0) win = cands[best];
                 }
                 (void)hipStreamSynchronize(s);
-                (void)hipFree(dt);
-                // As in the plans' race: 1.5% and 0.1 us, or the earlier preset stays.
-                if (good && (best > 1e29 || kt < 0.985 * best - 1e-4)) {
-                    best = kt;
-                    win = k;
-                }
             }
+            (void)hipStreamDestroy(s);
         }
-        if (have_e1) (void)hipEventDestroy(e1);
-        if (have_e0) (void)hipEventDestroy(e0);
-        if (have_s) (void)hipStreamDestroy(s);
+        for (int2* t : tasks) (void)hipFree(t);
         std::memcpy(m->batch, saved, sizeof saved);
     }
     for (void* b : bufs) (void)hipFree(b);

@@ -28,6 +28,7 @@
 #include "cx.hpp"
 #include "fft3d_mi355x.h"
 #include "plan_internal.hpp"
+#include "race_hip.hpp"
 #include "registry.hpp"
 
 namespace fx {
@@ -98,107 +99,6 @@ static std::string wisdom_key(int n0, int n1, int n2, int prec, int dir, long ba
     return buf;
 }
 
-// One candidate of a race, launched in groups of n between two events, n chosen so that a group
-// lasts about 300 us (5..64), 1.5 ms in the final: event timing jitter of a few microseconds
-// would otherwise decide between kernels of ~10 us.  Successive launches use successive windows of the race buffers,
-// so with enough windows no launch finds its data in the 256 MB Infinity Cache and the race
-// ranks kernels as they run from HBM.
-struct Trial {
-    const KernelDesc* k;
-    int n;        // launches per group; 0: failed to launch, or out of the race
-    int warm;     // launches before a group that are not timed
-    double best;  // fastest group, seconds per launch
-};
-
-struct RaceRig {
-    const char* din;
-    char* dout;
-    size_t wbytes;
-    int nwin;
-    long nvol;
-    const void* bank;
-    unsigned* work;
-    hipStream_t s;
-    std::vector<hipEvent_t> ev;   // two per candidate
-    int w = 0;
-
-    bool launch(const KernelDesc& k, int n)
-    {
-        for (int i = 0; i < n; ++i) {
-            const size_t off = (size_t)(w++ % nwin) * wbytes;
-            if (k.launch(din + off, dout + off, nvol, bank, 1.0, work, s) != hipSuccess) return false;
-        }
-        return true;
-    }
-    // One group of every candidate still in the race, one after another on the stream with
-    // nothing waited for in between: seconds per launch into t (-1 where a launch failed).
-    bool round(const std::vector<Trial>& ts, std::vector<double>& t)
-    {
-        t.assign(ts.size(), -1.0);
-        size_t last = ts.size();
-        for (size_t i = 0; i < ts.size(); ++i) {
-            if (!ts[i].n) continue;
-            const bool warm = launch(*ts[i].k, ts[i].warm);
-            if (hipEventRecord(ev[2 * i], s) != hipSuccess) return false;
-            if (warm && launch(*ts[i].k, ts[i].n)) t[i] = 0.0;
-            if (hipEventRecord(ev[2 * i + 1], s) != hipSuccess) return false;
-            last = i;
-        }
-        if (last == ts.size() || hipEventSynchronize(ev[2 * last + 1]) != hipSuccess) return false;
-        for (size_t i = 0; i < ts.size(); ++i) {
-            if (t[i] != 0.0) continue;
-            float ms = 0.f;
-            if (hipEventElapsedTime(&ms, ev[2 * i], ev[2 * i + 1]) != hipSuccess) return false;
-            t[i] = (double)ms * 1e-3 / ts[i].n;
-        }
-        return true;
-    }
-};
-
-// Sizes every candidate's groups (which also brings the clocks up), then times the candidates
-// in turn, one group each a round, so that none has the cold or the busy end of the race to
-// itself: timed one after the other, kernels 5% apart changed places from run to run.  Two
-// rounds of short groups leave those within 25% and then 10% of the first; two rounds of longer
-// ones, each after some launches of the same kernel that are not timed, decide.  A kernel's
-// first launches run against what the kernel before it left in the caches: in groups of five a
-// persistent 6^3 complex128 kernel takes 74 us to a staged one's 77, and 79.5 to 77.6 in runs
-// of 40; at 17^3 x 2798 the order of two turns round likewise (88 : 91 and 90 : 87).
-static void run_trials(RaceRig& r, std::vector<Trial>& ts)
-{
-    std::vector<double> t;
-    auto size = [](double per, double group, int most) {
-        const int n = (int)(group / per);
-        return n < 5 ? 5 : n > most ? most : n;
-    };
-    for (Trial& c : ts) {
-        c.best = 1e30;
-        c.warm = 0;
-        c.n = r.launch(*c.k, 2) ? 5 : 0;
-    }
-    if (!r.round(ts, t)) return;
-    for (size_t i = 0; i < ts.size(); ++i) ts[i].n = t[i] > 0 ? size(t[i], 300e-6, 64) : 0;
-    const double keep[4] = {1.25, 1.10, 1.05, 1.05};
-    for (int round = 0; round < 4; ++round) {
-        if (round == 2)
-            for (Trial& c : ts) {
-                if (!c.n) continue;
-                c.n = size(c.best, 1.5e-3, 256);
-                c.warm = c.n / 3;
-                c.best = 1e30;
-            }
-        if (!r.round(ts, t)) return;
-        double lead = 1e30;
-        for (size_t i = 0; i < ts.size(); ++i) {
-            if (!ts[i].n) continue;
-            if (t[i] <= 0) ts[i].n = 0, ts[i].best = 1e30;
-            else if (t[i] < ts[i].best) ts[i].best = t[i];
-            if (ts[i].best < lead) lead = ts[i].best;
-        }
-        for (Trial& c : ts)
-            if (c.best > keep[round] * lead) c.n = 0, c.best = 1e30;
-    }
-}
-
 // *best_s = 0 when no trial completed (no race buffers, or every launch failed): the
 // first candidate is returned unmeasured and the caller must not record it as wisdom.
 static const KernelDesc* race(const std::vector<const KernelDesc*>& cands, int n0, int n1,
@@ -234,30 +134,35 @@ static const KernelDesc* race(const std::vector<const KernelDesc*>& cands, int n
     const KernelDesc* win = cands[0];
     double wt = 1e30;
     if (hipStreamCreate(&s) == hipSuccess) {
-        RaceRig rig{(const char*)din, (char*)dout, wbytes, nwin, rb, bank, work, s, {}};
-        for (size_t i = 0; i < 2 * cands.size(); ++i) {
-            hipEvent_t e;
-            if (hipEventCreate(&e) != hipSuccess) break;
-            rig.ev.push_back(e);
-        }
-        if (rig.ev.size() == 2 * cands.size()) {
-            std::vector<Trial> ts;
-            for (const KernelDesc* k : cands) ts.push_back(Trial{k, 0, 0, 1e30});
-            run_trials(rig, ts);
-            // A later candidate must beat the incumbent by more than 1.5% (above the
-            // run-to-run spread of one trial) and a tenth of a microsecond more, so near-ties
-            // resolve the same way each time, to the earlier-registered variant.  The tenth
-            // is for kernels that last as long as a launch: there a full queue hides a
-            // kernel's start, which a paced caller pays (6^3 complex128 x 289: 3.74 us here to
-            // the staged kernel's 3.82, and 4.5 to 3.9 launched from Python).
-            for (const Trial& t : ts)
-                if (t.best < 1e29 && (wt > 1e29 || t.best < 0.985 * wt - 0.1e-6)) {
-                    wt = t.best;
-                    win = t.k;
+        {
+            RaceEvents ev(cands.size());
+            // Successive launches use successive windows of the race buffers, so with enough of
+            // them no launch finds its data in the 256 MB Infinity Cache and the race ranks
+            // kernels as they run from HBM.
+            int w = 0;
+            auto launch = [&](size_t k, int n) {
+                for (int i = 0; i < n; ++i) {
+                    const size_t off = (size_t)(w++ % nwin) * wbytes;
+                    if (cands[k]->launch((const char*)din + off, (char*)dout + off, rb, bank, 1.0, work, s) !=
+                        hipSuccess)
+                        return false;
                 }
+                return true;
+            };
+            std::vector<Trial> ts(cands.size());
+            int best = -1;
+            if (ev.ok) {
+                run_trials(ts, kPlanRace, 0, launch, [&](const std::vector<Trial>& c, std::vector<double>& t) {
+                    return ev.round(c, t, s, launch);
+                });
+                best = race_winner(ts);
+            }
+            if (best >= 0) {
+                wt = ts[best].best;
+                win = cands[best];
+            }
+            (void)hipStreamSynchronize(s);
         }
-        (void)hipStreamSynchronize(s);
-        for (hipEvent_t e : rig.ev) (void)hipEventDestroy(e);
         (void)hipStreamDestroy(s);
     }
     (void)hipFree(din);
