@@ -97,7 +97,7 @@ static const MultiDesc* multi_race(fft3d_mx_multi* m, const std::vector<const Mu
     std::vector<void*> bufs;
     std::vector<std::vector<const void*>> ins(sets, std::vector<const void*>(m->nitems));
     std::vector<std::vector<void*>> outs(sets, std::vector<void*>(m->nitems));
-    auto alloc = [&] {
+    auto alloc = [&](int sets) {
         for (int i = 0; i < m->nitems; ++i) {
             const int g = m->code[i];
             rb[i] = std::max(m->batch[i] > 0 ? 1 : 0, (int)(m->batch[i] * shrink));
@@ -109,7 +109,11 @@ static const MultiDesc* multi_race(fft3d_mx_multi* m, const std::vector<const Mu
                              hipMalloc(&b, pitch * sets) == hipSuccess;
             if (a) bufs.push_back(a);
             if (b) bufs.push_back(b);
-            if (!got) return false;
+            if (!got) {
+                for (void* p : bufs) (void)hipFree(p);
+                bufs.clear();
+                return false;
+            }
             (void)hipMemsetD32((hipDeviceptr_t)a, 0x3F800000u, pitch * sets / 4);
             for (int w = 0; w < sets; ++w) {
                 ins[w][i] = (char*)a + w * pitch;
@@ -118,15 +122,9 @@ static const MultiDesc* multi_race(fft3d_mx_multi* m, const std::vector<const Mu
         }
         return true;
     };
-    bool ok = alloc();
-    if (!ok && sets > 1) {   // memory is short: one set
-        for (void* b : bufs) (void)hipFree(b);
-        bufs.clear();
-        sets = 1;
-        ok = alloc();
-    }
+    sets = fit_sets(sets, alloc);   // fewer where memory is short
     const MultiDesc* win = cands[0];
-    if (ok) {
+    if (sets > 0) {
         int saved[kMultiMaxItems];
         std::memcpy(saved, m->batch, sizeof saved);
         std::memcpy(m->batch, rb, sizeof(int) * m->nitems);

@@ -117,17 +117,16 @@ static const KernelDesc* race(const std::vector<const KernelDesc*>& cands, int n
     int nwin = (int)(((768ull << 20) + wbytes - 1) / wbytes);
     if (nwin > 8) nwin = 8;
     void *din = nullptr, *dout = nullptr;
-    for (; nwin >= 1; nwin = nwin > 1 ? nwin / 2 : 0) {
-        if (hipMalloc(&din, nwin * wbytes) != hipSuccess) {
-            din = nullptr;
-            continue;
+    nwin = fit_sets(nwin, [&](int n) {
+        if (hipMalloc(&din, n * wbytes) == hipSuccess) {
+            if (hipMalloc(&dout, n * wbytes) == hipSuccess) return true;
+            (void)hipFree(din);
         }
-        if (hipMalloc(&dout, nwin * wbytes) == hipSuccess) break;
-        (void)hipFree(din);
         din = dout = nullptr;
-    }
+        return false;
+    });
     (void)hipGetLastError();
-    if (!din || !dout) return cands[0];
+    if (!nwin) return cands[0];
     // 0x3F80_0000 per 32-bit word: 1.0f for complex64, ~0.0078 per double for complex128.
     (void)hipMemsetD32((hipDeviceptr_t)din, 0x3F800000u, nwin * wbytes / 4);
     hipStream_t s;

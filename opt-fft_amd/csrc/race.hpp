@@ -90,6 +90,16 @@ void run_trials(std::vector<Trial>& ts, const RaceRules& rules, int cycle, Launc
     }
 }
 
+// Sets of buffers that a race may use: alloc(n) for n = sets and then half as many each time, until
+// it succeeds (it keeps nothing where it fails).  0 if not even one was had.
+template <class Alloc>
+int fit_sets(int sets, Alloc alloc)
+{
+    for (; sets >= 1; sets /= 2)
+        if (alloc(sets)) return sets;
+    return 0;
+}
+
 // The candidate a race picked, -1 if none ran to the end.  A later one must beat the incumbent by
 // more than 1.5% (above the run-to-run spread of one trial) and a tenth of a microsecond more,
 // so near-ties resolve the same way each time, to the earlier-registered variant.  The tenth is

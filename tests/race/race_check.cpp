@@ -87,6 +87,18 @@ int main()
     CHECK(mix.race(kMultiRace, 2) == 7);
     printf("large mix: %d launches, %.1f ms\n", mix.launches, mix.spent * 1e-3);
     CHECK(mix.spent <= 12.7e3);
+    // Short memory: as many sets as fit, by halves, with nothing kept of an attempt that failed.
+    for (int room = 0; room <= 40; ++room) {
+        int held = 0, tries = 0;
+        const int got = fit_sets(16, [&](int n) {
+            ++tries;
+            held = n <= room ? n : 0;
+            return held > 0;
+        });
+        int most = 16;
+        while (most > room) most /= 2;
+        CHECK(got == most && held == got && tries <= 5);
+    }
     printf("OK\n");
     return 0;
 }
