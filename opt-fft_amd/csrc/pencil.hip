@@ -211,8 +211,6 @@ void register_pencil(std::vector<KernelDesc>& r)
     FX_X_BOTH(24, 24, 24, float, "c64", 2, 320, 2);
     FX_X_BOTH(24, 24, 24, float, "c64", 3, 192, 4);
     FX_X_BOTH(24, 24, 24, float, "c64", 6, 192, 6);
-#define TT(N0,N1,N2,T,TAG,R,NT,PR,GS,PF,LIN) \
-    r.push_back(xhold_desc<XHoldCfg<N0,N1,N2,T,-1,R,NT,PR,GS,PF,LIN>>("T" #N0 "x" #N1 "x" #N2 TAG "r" #R "t" #NT "h" #PR "g" #GS "f" #PF "l" #LIN));
     FX_XH_BOTH(36, 36, 36, double, "c128", 2, 256, 6, 9, 3);
     FX_XH_BOTH(36, 36, 36, double, "c128", 4, 448, 6, 9, 2);
     FX_XH_BOTH(24, 24, 48, double, "c128", 2, 256, 8, 6, 4);
