@@ -109,7 +109,7 @@ namespace fx {
 void register_pencil(std::vector<KernelDesc>& r)
 {
     // L = 36: slab 36x36 = 20.7 KB complex128.  The race keeps an earlier variant unless a
-    // later one is >2% faster: at batch 128 s7t256p1 staggered (71 us), then unstaggered
+    // later one is 1.5% and 0.1 us faster: at batch 128 s7t256p1 staggered (71 us), then unstaggered
     // (73 us), ahead of s3t128p2 (73-74 us).
     FX_PS_BOTH(36, 36, 36, double, "c128", 7, 256, 1, 128, 0, 1);
     FX_P_BOTH(36, 36, 36, double, "c128", 7, 256, 1, 128, 0, 1);
@@ -219,6 +219,9 @@ void register_pencil(std::vector<KernelDesc>& r)
     FX_XH_BOTH(24, 24, 24, float, "c64", 1, 192, 8, 6, 4);
     FX_XHL_BOTH(24, 24, 24, float, "c64", 1, 192, 8, 6, 4);
     FX_XHL_BOTH(36, 36, 36, float, "c64", 1, 448, 12, 9, 4);
+    // 256 threads, 6 planes in LDS and 12 held: ahead of the other single forms at 36^3 complex64 x
+    // 300-384 (66.8-68.4 us; r1h12l 69.2-72.2, r2h9l 70.2-73.6) and nowhere the quickest, since the
+    // rounds take 58.4-66.5 there; between 40 and 256 volumes r2h9l or r1h12l is 10% ahead.
     FX_XHL_BOTH(36, 36, 36, float, "c64", 2, 256, 6, 9, 4);
     FX_XHL_BOTH(36, 36, 36, float, "c64", 2, 448, 9, 9, 3);
 }

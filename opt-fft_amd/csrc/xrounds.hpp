@@ -1,7 +1,7 @@
-// Residue-split launch by rounds.  A form (a residue-split kernel with R workgroups a volume,
-// W of them on a CU) takes about as long for one volume as for a device full of them, and as
-// long again for the next one: 36^3 complex128 in two workgroups a volume takes 27.7 us for 1
-// volume, 41.5 for 128 (one round of 256 workgroups), 70.4 for 150 and 80.0 for 256.  Fewer
+// Residue-split launch by rounds.  A form (a residue-split kernel with R workgroups a volume)
+// takes about as long for one volume as for a round of them, and as long again for the next one:
+// 36^3 complex128 in two workgroups a volume takes 27.7 us for 1 volume, 41.5 for 128 (one round
+// of 256 workgroups), 70.4 for 150 and 80.0 for 256.  Fewer
 // volumes than a round go faster through a form with more workgroups a volume, as long as
 // those run in one round themselves.  So a batch runs its full rounds in the last form of the
 // list, and what remains in the first form (R descending) that holds it in one round, as a
@@ -9,6 +9,12 @@
 //   36^3 complex128, 2 / 4 / 6 / 12 workgroups a volume, rounds of 128 / 64 / 40 / 16 volumes:
 //   16 volumes 32.1 / 22.0 / 14.8 / 13.5 us, 32 volumes 32.6 / 22.7 / 17.4 / 24.4,
 //   64 volumes 34.3 / 26.7 / 33.2 / 35.7, 128 volumes 41.5 / 51.9 / 57.1 / 69.7.
+// W of a form is the number of workgroups a CU that its round is counted with, where its time was
+// measured to step: not its occupancy, which is higher for most (LDS alone would let two
+// workgroups of 24^3 complex128 r4 share a CU, but 80 volumes take 14.4 us to the 8.9 of 64; 40
+// volumes of r6 7.1 us, 56 12.4).  24^3 complex64 r1h8 steps after 512 volumes, W = 2 (22.6 us; 600
+// 31.4), and the same form with linear stores is ahead from there on (23.9 and 30.0): it ends the
+// list with the four workgroups that fit on a CU.
 // Where the last form has several workgroups on a CU (W > 1) its rounds overlap, and a batch of
 // more than one of them runs in that form alone: 24^3 complex64 x 1200 took 56.6 us in two
 // launches and 55.5 in one, 24^3 complex128 x 340 35.9 and 31.5.
@@ -22,7 +28,7 @@ namespace fx {
 
 constexpr int kXcds = 8;
 
-// Volumes of one round of R workgroups a volume, W workgroups a CU.
+// Volumes of one round of R workgroups a volume, counted with W workgroups a CU.
 inline long round_volumes(int cus, int R, int W) { return (long)(cus / kXcds * W / R) * kXcds; }
 
 template <class C_, int W_>
