@@ -23,7 +23,6 @@ void register_multi(std::vector<MultiDesc>& r)
     r.push_back(multi_desc<float, 4>("multi_c64_t320_fill_lin_mix", 1));
     r.push_back(multi_desc<float, 4>("multi_c64_t320_fill_lin"));
     r.push_back(multi_desc<double, 5>("multi_c128_t640_lin"));
-    r.push_back(multi_desc<double, 5>("multi_c128_t640_lin_mix", 1));
     r.push_back(multi_desc<double, 6>("multi_c128_t192"));
     r.push_back(multi_desc<double, 7>("multi_c128_t192_lin"));
     r.push_back(multi_desc<float, 8>("multi_c64_t320_lin"));

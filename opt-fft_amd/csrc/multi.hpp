@@ -119,7 +119,9 @@ struct MultiPreset<T, 5> : LinPreset<T, 1, 0> {};
 // small geometries hold most of the bytes, 6^3 x 10000, 8^3 x 4000, 12^3 x 1500, 17^3 x 500
 // 65.7 -> 61.2, and 9 at complex64, 12^3 x 4854 with 17^3 x 258 36.3 -> 35.7; 8x8x16 x 6000 with
 // 17^3 x 100 takes 58.2 (54.4 as preset 3).  Not registered: 6 and 7 with the items interleaved
-// (127-140 us in place of 61-68 at the mix above), 9 at complex128 (two workgroups a CU: 42.0
+// (127-140 us in place of 61-68 at the mix above), 5 interleaved (behind t640_mix or a 192-thread
+// preset in each of eleven mixes, 66.7 to 61.9 at the same one, 17^3 x 1000 with 8^3 x 16000 91.7 to
+// 81.9), 9 at complex128 (two workgroups a CU: 42.0
 // to 31.0 at 6^3 with 8^3), 192 threads at complex64 (within 2% of 8).
 template <typename T>
 struct MultiPreset<T, 6> {
