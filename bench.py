@@ -37,7 +37,9 @@ within 2 ms, for continuous batching and for the two plain one-launch-per-reques
 throughput ratio of batching to each at that cap, and each mode's results checked on a
 sampled burst against numpy.fft.
 
-Prints ONE JSON line.  `python bench.py --gpus N` with N > 1 exits: the benchmark runs on one
+Prints ONE JSON line: the contract's fields and of the rest the figures (BRIEF), under 7,000 bytes,
+so that whoever keeps only the end of the output has the whole of it.  --record PATH writes the
+full record, every load point, window and candidate, as JSON.  `python bench.py --gpus N` with N > 1 exits: the benchmark runs on one
 GPU (batches of independent volumes shard by volume with no communication).
 """
 import argparse
@@ -614,6 +616,30 @@ def host_abi(pkg, L=17, batch=1024, reps=8):
                     "and copies out per execute, pipelined in ~8 MB chunks; not `value`"}
 
 
+# What the printed line keeps of each block.
+BRIEF = {
+    "cpu_baseline": ("value", "unit", "cores", "kind", "sample"),
+    "secondary": ("kernel", "ms_per_execute", "transforms_per_s", "roofline_frac", "rel_l2_vs_numpy"),
+    "precision_variants": ("kernel", "us", "rel_l2"),
+    "small_batch_latency": ("kernel", "device_us_per_execute", "round_trip_us_median"),
+    "host_abi": ("ms_per_execute", "transforms_per_s", "rel_l2_vs_numpy"),
+    "serving": ("max_rate_req_s", "p50_ms", "p99_ms", "transforms_per_s", "c128", "c64",
+                "throughput_ratio_vs_plain_at_p99_cap", "throughput_ratio_vs_plain_async_at_p99_cap"),
+}
+
+
+def brief(record):
+    """The printed line: the record with the blocks of BRIEF cut to the leaves named there (at any
+    depth) and their figures to five digits."""
+    def cut(v, keys):
+        if isinstance(v, dict):
+            kept = {k: cut(x, keys) for k, x in v.items()
+                    if k in keys or isinstance(x, dict)}
+            return {k: x for k, x in kept.items() if x != {}}
+        return float(f"{v:.5g}") if isinstance(v, float) else v
+    return {k: cut(v, BRIEF[k]) if k in BRIEF and v is not None else v for k, v in record.items()}
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -622,6 +648,7 @@ def main():
     ap.add_argument("--windows", type=int, default=5,
                     help="timed windows after the contract region (the value is their median)")
     ap.add_argument("--window-ms", type=float, default=20.0, help="minimum window length")
+    ap.add_argument("--record", default=None, metavar="PATH", help="write the full record there")
     ap.add_argument("--no-secondary", action="store_true")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-serving", action="store_true")
@@ -712,7 +739,10 @@ def main():
         "host_abi": habi,
         "serving": serve,
     }
-    print(json.dumps(line), flush=True)
+    if a.record:
+        with open(a.record, "w") as out:
+            json.dump(line, out, indent=1)
+    print(json.dumps(brief(line)), flush=True)
 
 
 if __name__ == "__main__":
