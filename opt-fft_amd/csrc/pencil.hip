@@ -135,29 +135,24 @@ void register_pencil(std::vector<KernelDesc>& r)
     FX_PR_BOTH(24, 24, 24, double, "c128", 8, 192, 1, 128, 0, 2, 0, "");
     FX_P_BOTH(24, 24, 48, float, "c64", 8, 384, 1, 128, 0, 2);
     FX_P_BOTH(24, 24, 48, float, "c64", 8, 256, 1, 128, 0, 0);
-    // Residue-split single pass (forced by name, rotated buffers, medians of >= 25 ms
-    // windows).  36^3 x 128: r6 (127.9 KB, one workgroup per CU) 64.6 us with 512 threads,
-    // 65.3 with 256, against 66.9 us for the best pencil; r12 (63.9 KB, two per CU, 12 reads
-    // of every element from L2) 84.7 us.  24x24x48 x 64: r4 (112.9 KB) 16.9 us with 384
-    // threads, 18.2 with 256, against 22.5 us; r6 / r8 (two per CU) 23.1 / 22.6 us.  24^3 x 512:
-    // r3 (76.8 KB, two per CU) 46.1 us with 256 threads, 48.5 with 192; r2 50.2, r4 55.8-56.1,
-    // against 53.3 us for the split-resident kernel; at batch 64 r4 / r3 10.4 / 10.5 us
-    // against 16.1 us for the pencil.  Thread counts keep every variant within its VGPR
+    // Residue-split single pass (forced by name, over 1 GB of buffers in turn).  24x24x48 x 64: r4
+    // (112.9 KB) 16.6-16.8 us with 384 threads, 17.2 with 256, r8 18.8, against 22.5 us for the best
+    // pencil; 24^3 x 512: r3 (76.8 KB, two per CU) 45.6 us with 256 threads, 46.2 with 192, r4 52.6,
+    // against 53.2 us for the split-resident kernel; x 64 r4 8.9, r3 9.1 against 15.7 us for the
+    // pencil, x 8 r6 6.0, r4 6.6, r3 7.0.  36^3 x 128: r6 (127.9 KB, one workgroup per CU) 55.6 us,
+    // r12 (63.9 KB, 12 reads of every element from L2) 68.4, against 67.0 us for the best pencil
+    // and 40.3 with held planes (xhold.hpp).  Thread counts keep every variant within its VGPR
     // budget without scratch (a 48-point complex128 line takes ~200 VGPRs).  Point order
-    // of the x pass (one device): 36^3 x 128 57.1 us with offset starts (o2), 57.5 rotated
-    // blocks (o1), 65.2 from point 0; 24x24x48 x 64 16.6 (o2) against 17.6 us; 24^3 x 512
-    // 48.0 (o1) against 49.8 us; 36^3 complex64 x 64 19.8 (o2) against 20.6 us; 24x24x48
-    // complex64 x 256 30.0 (o2) against 29.1 us, not registered.  At 36^3 a
-    // workgroup's x pass (reading 746 KB from L2 at ~52 GB/s per CU) takes 14.4 us of its
-    // ~20 us; a persistent form computing the next task's x pass into registers during the
+    // of the x pass: 36^3 x 128 r6 57.4 us with offset starts (o2), 55.6 with rotated
+    // blocks (o1), 64.0 from point 0, x 1024 426 / 417 / 468; 36^3 complex64 x 64 r3 19.6 (o2) against
+    // 20.0; 24x24x48 x 64 16.9 / 16.6 / 16.8; 24^3 x 512 47.2 (o1) against 45.6, but x 64 9.2 both.
+    // Not kept, before the x pass was pipelined (xres.hpp): a persistent form at 36^3 that computes
+    // the next task's x pass into registers during the
     // LDS passes (256 threads, 486 VGPRs) ran at 165 us: at that register pressure its loads
     // were issued one or two at a time, and issuing them together spilled.  A second form
     // (512 threads, 169 VGPRs: two-stage 4 x 9 line passes, loads six at a time, offset
     // starts) ran without scratch but took 69.8 us at x 128 and 251.4 at x 512 against 57.0 /
-    // 225.3 us for the one-task form.  Not kept.  (The figures above are from before the x
-    // pass was pipelined, xres.hpp; since then 24x24x48 x 64 takes 16.4 us with rotated blocks
-    // (o1) and 16.7 with offset starts, and 24^3 x 8 6.0 us in six workgroups (r6) against 6.6
-    // in four, which is the better one from x 64 on.)
+    // 225.3 us for the one-task form.
     // By rounds, ahead of the single forms so that a plan that ties takes the launch that also
     // fits its smaller executes (single form -> by rounds, us):
     //   36^3              x 1 27.7 -> 11.3, x 64 34.2 -> 26.4, x 150 70.0 -> 57.0, x 258 107 -> 92
